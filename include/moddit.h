@@ -96,6 +96,31 @@ int moddit_block_sparse_fwd(const void* q, const void* k, const void* v, void* o
                             int grid_origin, moddit_stream_t stream);
 
 /*
+ * The two calls above with a device workspace (16-byte aligned, used on `stream` only, its
+ * contents undefined before and after). Launches with too few query tiles to fill the GPU
+ * then split each tile's key range over several workgroups, which leave fp32 partial
+ * results in the workspace, and combine them in a second launch. *_workspace_bytes gives
+ * the size such a call needs, 0 where it would not split; with a NULL workspace the calls
+ * are the plain ones. The results differ from the plain call's by fp32 summation order.
+ */
+int64_t moddit_flash_fwd_workspace_bytes(int batch, int heads, int q_len, int kv_len, int head_dim);
+int64_t moddit_block_sparse_fwd_workspace_bytes(int batch, int heads, int q_len, int head_dim,
+                                                int cap, int grid_origin);
+int moddit_flash_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                        int batch, int heads, int q_len, int kv_len, int head_dim,
+                        const int64_t q_strides[3], const int64_t k_strides[3],
+                        const int64_t v_strides[3], const int64_t o_strides[3],
+                        float softmax_scale, int dtype, void* workspace, int64_t workspace_bytes,
+                        moddit_stream_t stream);
+int moddit_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                               int batch, int heads, int q_len, int kv_len, int head_dim,
+                               const int64_t q_strides[3], const int64_t k_strides[3],
+                               const int64_t v_strides[3], const int64_t o_strides[3],
+                               float softmax_scale, int dtype, const int32_t* counts,
+                               const int32_t* entries, int n_qtiles, int cap, int grid_origin,
+                               void* workspace, int64_t workspace_bytes, moddit_stream_t stream);
+
+/*
  * Dense attention and the replayed sparsity map in one kernel: every workgroup runs
  * the dense pass of moddit_flash_fwd for its 128 query rows (O, and LSE when lse is not
  * NULL), then, with the rows' final LSE still in registers, sweeps the video key tiles

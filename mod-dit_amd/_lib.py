@@ -34,6 +34,14 @@ _SIGNATURES = {
     "moddit_block_sparse_fwd": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i,
                                      _c_i64p, _c_i64p, _c_i64p, _c_i64p, _f, _i,
                                      _vp, _vp, _i, _i, _i, _vp]),
+    "moddit_flash_fwd_workspace_bytes": (ctypes.c_int64, [_i, _i, _i, _i, _i]),
+    "moddit_flash_fwd_ws": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i,
+                                 _c_i64p, _c_i64p, _c_i64p, _c_i64p, _f, _i,
+                                 _vp, ctypes.c_int64, _vp]),
+    "moddit_block_sparse_fwd_workspace_bytes": (ctypes.c_int64, [_i, _i, _i, _i, _i, _i]),
+    "moddit_block_sparse_fwd_ws": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i,
+                                        _c_i64p, _c_i64p, _c_i64p, _c_i64p, _f, _i,
+                                        _vp, _vp, _i, _i, _i, _vp, ctypes.c_int64, _vp]),
     "moddit_flash_fwd_map": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i,
                                   _c_i64p, _c_i64p, _c_i64p, _c_i64p, _f, _f, _i, _i, _i, _i,
                                   _vp]),

@@ -76,6 +76,10 @@ struct AttnParams {
   int map_valid;     // video tokens that exist: min(map_nblk*map_block, seq_len - map_q_off)
   float map_scale;   // softmax scale applied to q before rounding
   float map_log_thr; // ln(threshold)
+  // split key range (kSplit kernels): `n_split` workgroups per query tile
+  int n_split;
+  float* part_o;   // [tile][piece][128][D]: unnormalised O of the piece, relative to its max
+  float* part_ml;  // [tile][piece][128][2]: running max (log2 units) and row sum
 };
 
 // K rows are stored in LDS in the order pi(r): inside every 16-row chunk the row groups
@@ -109,7 +113,9 @@ __device__ __forceinline__ s16x4 lds_read_tr16(const unsigned char* a) {
 constexpr int kMapFlush = 64;
 constexpr int kMapCountBytes = 4 * 2 * kMapFlush * 4;  // int per (wave, ring slot)
 
-template <int D, typename E, bool kSparse, bool kRagged, bool kMap = false>
+// kSplit: one workgroup takes the piece `blockIdx % n_split` of a query tile's key tiles (or
+// list entries) and leaves its unnormalised fp32 O, max and sum for combine_kernel.
+template <int D, typename E, bool kSparse, bool kRagged, bool kMap = false, bool kSplit = false>
 __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_fwd_kernel(AttnParams p) {
   using L = AttnLds<D>;
   using V8 = typename E::vec8;
@@ -127,7 +133,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   const int half = lane >> 5;
   const int c32 = lane & 31;
 
-  const int tile = xcd_remap(blockIdx.x, gridDim.x, p.xcd_run);
+  const int tile = kSplit ? blockIdx.x / p.n_split : xcd_remap(blockIdx.x, gridDim.x, p.xcd_run);
   const int qt = tile % p.n_qtiles;
   const int bh = tile / p.n_qtiles;
   const int b = bh / p.heads;
@@ -146,6 +152,16 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     list = p.entries + slot * p.cap;
   } else {
     n_iter = p.n_ktiles;
+  }
+  int it0 = 0;  // first key tile (dense) of this workgroup's piece
+  if constexpr (kSplit) {
+    const int piece = blockIdx.x - tile * p.n_split;
+    const int first = static_cast<int>(static_cast<int64_t>(n_iter) * piece / p.n_split);
+    n_iter = static_cast<int>(static_cast<int64_t>(n_iter) * (piece + 1) / p.n_split) - first;
+    if (kSparse)
+      list += first;
+    else
+      it0 = first;
   }
   const int wbit = 1 << (wave >> 1);
 
@@ -243,7 +259,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     flags = (kt >= 0 && kt < p.n_ktiles) ? (e & 3) : 0;
     kt = kt < 0 ? 0 : (kt < p.n_ktiles ? kt : p.n_ktiles - 1);
   };
-  auto entry = [&](int i) -> int { return kSparse ? list[i] : ((i << 2) | 3); };
+  auto entry = [&](int i) -> int { return kSparse ? list[i] : (((it0 + i) << 2) | 3); };
 
   auto qk = [&](const unsigned char* ks, f32x16& s0, f32x16& s1) {
     s0 = f32x16{};
@@ -395,6 +411,21 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
 
   // ---- epilogue ----
   const float l_tot = sum_over_halves(l_run);
+  if constexpr (kSplit) {
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * kBM + wave * 32 + c32;
+    float* po = p.part_o + row * D;
+#pragma unroll
+    for (int dsub = 0; dsub < kDSub; ++dsub)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(po + dsub * 32 + 8 * g + 4 * half) =
+            f32x4{oacc[dsub][4 * g], oacc[dsub][4 * g + 1], oacc[dsub][4 * g + 2], oacc[dsub][4 * g + 3]};
+    if (half == 0) {
+      p.part_ml[2 * row] = m_run;
+      p.part_ml[2 * row + 1] = l_tot;
+    }
+    return;
+  }
   if (q_row >= 0 && q_row < p.q_len) {
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     uint16_t* orow = p.o + b * p.o_sb + h * p.o_sh + q_row * p.o_ss;
@@ -529,10 +560,53 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   }
 }
 
-template <int D, typename E, bool kSparse, bool kRagged, bool kMap = false>
+// The pieces of a query tile -> its rows of O and LSE: with m the largest of the pieces'
+// maxima, O = sum_i 2^(m_i - m) O_i / sum_i 2^(m_i - m) l_i, in fp32 and in piece order
+// (deterministic). Bound by reading the partials back, mostly from L2 and the last-level
+// cache. A workgroup takes kCombineRows rows of one tile, a thread four of its columns.
+constexpr int kCombineRows = 16;
+
+template <int D, typename E>
+__global__ __launch_bounds__(kThreads) void combine_kernel(AttnParams p) {
+  constexpr int kCols = D / 4;  // threads per row
+  constexpr int kRowsPerPass = kThreads / kCols;
+  const int tile = blockIdx.x / (kBM / kCombineRows);
+  const int r_first = (blockIdx.x % (kBM / kCombineRows)) * kCombineRows;
+  const int qt = tile % p.n_qtiles;
+  const int bh = tile / p.n_qtiles;
+  const int b = bh / p.heads;
+  const int h = bh - b * p.heads;
+  const int d = (threadIdx.x % kCols) * 4;
+  for (int r = r_first + threadIdx.x / kCols; r < r_first + kCombineRows; r += kRowsPerPass) {
+    const int q_row = p.origin + qt * kBM + r;
+    if (q_row < 0 || q_row >= p.q_len) continue;
+    const int64_t row0 = static_cast<int64_t>(tile) * p.n_split * kBM + r;
+    float m = -INFINITY;
+    for (int i = 0; i < p.n_split; ++i) m = fmaxf(m, p.part_ml[2 * (row0 + i * kBM)]);
+    const float m_use = m == -INFINITY ? 0.f : m;
+    float l = 0.f;
+    f32x4 o = f32x4{};
+    for (int i = 0; i < p.n_split; ++i) {
+      const int64_t row = row0 + i * kBM;
+      const float w = __builtin_amdgcn_exp2f(p.part_ml[2 * row] - m_use);
+      l += p.part_ml[2 * row + 1] * w;
+      o += *reinterpret_cast<const f32x4*>(p.part_o + row * D + d) * w;
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    u32x2 w2;
+    w2.x = pack2(E::from_float(o[0] * inv), E::from_float(o[1] * inv));
+    w2.y = pack2(E::from_float(o[2] * inv), E::from_float(o[3] * inv));
+    *reinterpret_cast<u32x2*>(p.o + b * p.o_sb + h * p.o_sh + q_row * p.o_ss + d) = w2;
+    if (p.lse != nullptr && d == 0)
+      p.lse[static_cast<int64_t>(bh) * p.q_len + q_row] =
+          l > 0.f ? (m + log2f(l)) * 0.69314718055994531f : -INFINITY;
+  }
+}
+
+template <int D, typename E, bool kSparse, bool kRagged, bool kMap = false, bool kSplit = false>
 int launch_attention_impl(const AttnParams& p, int batch, hipStream_t stream) {
   using L = AttnLds<D>;
-  auto kernel = attention_fwd_kernel<D, E, kSparse, kRagged, kMap>;
+  auto kernel = attention_fwd_kernel<D, E, kSparse, kRagged, kMap, kSplit>;
   constexpr int kLds = L::kTotal + (kMap ? kMapCountBytes : 0);
   static LaunchSetup once;
   if (set_dynamic_lds_once(once, reinterpret_cast<const void*>(kernel), kLds) != hipSuccess) {
@@ -541,12 +615,18 @@ int launch_attention_impl(const AttnParams& p, int batch, hipStream_t stream) {
   }
   const int64_t tiles = static_cast<int64_t>(batch) * p.heads * p.n_qtiles;
   if (tiles == 0) return MODDIT_OK;
-  if (tiles > 0x7fffffff) {
+  const int64_t grid = kSplit ? tiles * p.n_split : tiles;
+  if (grid > 0x7fffffff) {
     set_error("attention: too many tiles (%lld)", static_cast<long long>(tiles));
     return MODDIT_EINVAL;
   }
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), kLds, stream, p);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kThreads), kLds, stream, p);
   MODDIT_CHECK_LAUNCH("attention");
+  if constexpr (kSplit) {
+    hipLaunchKernelGGL((combine_kernel<D, E>), dim3(static_cast<unsigned>(tiles * (kBM / kCombineRows))),
+                       dim3(kThreads), 0, stream, p);
+    MODDIT_CHECK_LAUNCH("attention (combine)");
+  }
   return MODDIT_OK;
 }
 
@@ -555,12 +635,78 @@ int launch_attention(const AttnParams& p, int batch, hipStream_t stream) {
   // The fused map pass addresses video key tiles that may extend past the last key
   // (partial last block): always the range-checked path.
   if (p.map != nullptr) return launch_attention_impl<D, E, false, true, true>(p, batch, stream);
+  // The split kernel exists in the range-checked form only (its masking is one scalar test
+  // per key tile).
+  if (p.n_split > 1) return launch_attention_impl<D, E, kSparse, true, false, true>(p, batch, stream);
   // Key counts that are a multiple of the tile (on an unshifted grid) need no clamping
   // or masking at all.
   if (p.kv_len % kBN == 0 && p.origin == 0)
     return launch_attention_impl<D, E, kSparse, false>(p, batch, stream);
   return launch_attention_impl<D, E, kSparse, true>(p, batch, stream);
 }
+
+// ---- how many pieces a query tile's key range is split into ----
+// A launch of one workgroup per query tile leaves CUs idle when it has few tiles (a text
+// tail, a short clip, few heads): its time is a whole key sweep however few they are. The
+// sweep is then split over `n_split` workgroups per tile, at the price of writing and
+// re-reading fp32 partial outputs and one more launch. The choice compares estimates of
+// both, from the time a key tile takes with k workgroups on a CU (measured: D = 128
+// 1.48 / 2.18 / 3.49 / 4.20 us, D = 64 1.11 / 1.45 / 2.06 / 2.53 us for k = 1..4, and
+// 1.04 k and 0.61 k beyond). List lengths are known on the device only: a block-sparse
+// list is taken to hold a quarter of its capacity. Against the best of 1..32 pieces the
+// choice is within 5 % over 21 shapes; e.g. 256 text rows x 24 heads over 29,019 keys, D =
+// 128 (48 tiles): 650 us unsplit, 136 us in 10 pieces; over 115,419 keys 2,551 and 492 us;
+// 4,096 tokens x 2 heads, D = 64 (64 tiles): 70 and 30 us. From about one tile per CU on
+// the split no longer pays (432 tiles of 36 key tiles: 39 us unsplit, 59 us in two).
+constexpr int kMaxSplit = 64;
+// Key tiles per piece at the least: below 16 key tiles the second launch costs a dense call
+// what the split saves. A list's estimate is rough: real lists
+// hold a tenth to all of their capacity.
+constexpr int kMinPieceDense = 8;
+constexpr int kMinPieceSparse = 4;
+
+double cu_tile_us(int head_dim, int64_t k) {
+  if (head_dim == 128) return 1.05 * k + (k % 2 ? 0.38 : 0.08);
+  return 0.61 * k + (k == 1 ? 0.5 : 0.2);
+}
+
+int split_for(int64_t tiles, int64_t key_tiles, int min_piece, int head_dim) {
+  constexpr double kCus = 256, kFixedTiles = 2.5, kLaunchUs = 4.0, kPartialBytesPerUs = 4.0e6;
+  int best = 1;
+  double best_us = 0.0;
+  for (int s = 1; s <= kMaxSplit; ++s) {
+    if (s > 1 && key_tiles < static_cast<int64_t>(s) * min_piece) break;
+    const int64_t per_cu = static_cast<int64_t>((tiles * s + kCus - 1) / kCus);
+    double us = cu_tile_us(head_dim, per_cu) * (static_cast<double>(key_tiles) / s + kFixedTiles);
+    if (s > 1) us += kLaunchUs + tiles * s * (kBM * (head_dim + 2) * 8.0) / kPartialBytesPerUs;
+    if (s == 1 || us < 0.95 * best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+int64_t q_tiles_of(int q_len, int origin) { return (static_cast<int64_t>(q_len) - origin + kBM - 1) / kBM; }
+
+int dense_split(int batch, int heads, int q_len, int kv_len, int head_dim) {
+  return split_for(static_cast<int64_t>(batch) * heads * q_tiles_of(q_len, 0),
+                   (static_cast<int64_t>(kv_len) + kBN - 1) / kBN, kMinPieceDense, head_dim);
+}
+
+int sparse_split(int batch, int heads, int q_len, int head_dim, int origin, int cap) {
+  return split_for(static_cast<int64_t>(batch) * heads * q_tiles_of(q_len, origin), cap / 4,
+                   kMinPieceSparse, head_dim);
+}
+
+int64_t split_workspace_bytes(int64_t tiles, int n_split, int head_dim) {
+  return n_split > 1 ? tiles * n_split * kBM * (head_dim + 2) * static_cast<int64_t>(sizeof(float)) : 0;
+}
+
+struct SplitArgs {
+  void* workspace;
+  int64_t bytes;
+};
 
 struct MapArgs {
   void* out;
@@ -574,7 +720,8 @@ int attention_entry(const void* q, const void* k, const void* v, void* o, float*
                     int heads, int q_len, int kv_len, int head_dim, const int64_t* qs,
                     const int64_t* ks, const int64_t* vs, const int64_t* os, float scale,
                     int dtype, const int32_t* counts, const int32_t* entries, int n_qtiles,
-                    int cap, int origin, moddit_stream_t stream, const MapArgs* map = nullptr) {
+                    int cap, int origin, moddit_stream_t stream, const MapArgs* map = nullptr,
+                    const SplitArgs* split = nullptr) {
   clear_error();
   MODDIT_CHECK_ARG(q && k && v && o, "attention: null tensor pointer");
   MODDIT_CHECK_ARG(qs && ks && vs && os, "attention: null stride array");
@@ -665,6 +812,22 @@ int attention_entry(const void* q, const void* k, const void* v, void* o, float*
     }
   }
 
+  p.n_split = 1;
+  if (split != nullptr && split->workspace != nullptr) {
+    const int n_split = sparse ? sparse_split(batch, heads, q_len, head_dim, origin, cap)
+                               : dense_split(batch, heads, q_len, kv_len, head_dim);
+    const int64_t tiles = static_cast<int64_t>(batch) * heads * nq;
+    const int64_t need = split_workspace_bytes(tiles, n_split, head_dim);
+    MODDIT_CHECK_ARG(split->bytes >= need, "attention: workspace of %lld bytes, %lld needed",
+                     static_cast<long long>(split->bytes), static_cast<long long>(need));
+    MODDIT_CHECK_ARG(aligned16(split->workspace), "attention: workspace must be 16-byte aligned");
+    if (n_split > 1) {
+      p.n_split = n_split;
+      p.part_o = static_cast<float*>(split->workspace);
+      p.part_ml = p.part_o + tiles * n_split * kBM * head_dim;
+    }
+  }
+
   hipStream_t st = as_stream(stream);
   const bool bf = dtype == MODDIT_BF16;
   if (head_dim == 128) {
@@ -690,6 +853,53 @@ extern "C" int moddit_flash_fwd(const void* q, const void* k, const void* v, voi
   return moddit::attention_entry(q, k, v, o, lse, batch, heads, q_len, kv_len, head_dim,
                                  q_strides, k_strides, v_strides, o_strides, softmax_scale, dtype,
                                  nullptr, nullptr, 0, 0, 0, stream);
+}
+
+extern "C" int64_t moddit_flash_fwd_workspace_bytes(int batch, int heads, int q_len, int kv_len,
+                                                    int head_dim) {
+  using namespace moddit;
+  if (batch <= 0 || heads <= 0 || q_len <= 0 || kv_len <= 0) return 0;
+  return split_workspace_bytes(static_cast<int64_t>(batch) * heads * q_tiles_of(q_len, 0),
+                               dense_split(batch, heads, q_len, kv_len, head_dim), head_dim);
+}
+
+extern "C" int moddit_flash_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                                   int batch, int heads, int q_len, int kv_len, int head_dim,
+                                   const int64_t q_strides[3], const int64_t k_strides[3],
+                                   const int64_t v_strides[3], const int64_t o_strides[3],
+                                   float softmax_scale, int dtype, void* workspace,
+                                   int64_t workspace_bytes, moddit_stream_t stream) {
+  const moddit::SplitArgs split{workspace, workspace_bytes};
+  return moddit::attention_entry(q, k, v, o, lse, batch, heads, q_len, kv_len, head_dim,
+                                 q_strides, k_strides, v_strides, o_strides, softmax_scale, dtype,
+                                 nullptr, nullptr, 0, 0, 0, stream, nullptr, &split);
+}
+
+extern "C" int64_t moddit_block_sparse_fwd_workspace_bytes(int batch, int heads, int q_len,
+                                                           int head_dim, int cap, int grid_origin) {
+  using namespace moddit;
+  if (batch <= 0 || heads <= 0 || q_len <= 0 || cap <= 0 || grid_origin > 0 || grid_origin <= -kBN)
+    return 0;
+  return split_workspace_bytes(static_cast<int64_t>(batch) * heads * q_tiles_of(q_len, grid_origin),
+                               sparse_split(batch, heads, q_len, head_dim, grid_origin, cap), head_dim);
+}
+
+extern "C" int moddit_block_sparse_fwd_ws(const void* q, const void* k, const void* v, void* o,
+                                          float* lse, int batch, int heads, int q_len, int kv_len,
+                                          int head_dim, const int64_t q_strides[3],
+                                          const int64_t k_strides[3], const int64_t v_strides[3],
+                                          const int64_t o_strides[3], float softmax_scale,
+                                          int dtype, const int32_t* counts, const int32_t* entries,
+                                          int n_qtiles, int cap, int grid_origin, void* workspace,
+                                          int64_t workspace_bytes, moddit_stream_t stream) {
+  if (counts == nullptr) {
+    moddit::set_error("block_sparse_fwd: counts must not be NULL");
+    return MODDIT_EINVAL;
+  }
+  const moddit::SplitArgs split{workspace, workspace_bytes};
+  return moddit::attention_entry(q, k, v, o, lse, batch, heads, q_len, kv_len, head_dim,
+                                 q_strides, k_strides, v_strides, o_strides, softmax_scale, dtype,
+                                 counts, entries, n_qtiles, cap, grid_origin, stream, nullptr, &split);
 }
 
 extern "C" int moddit_flash_fwd_map(const void* q, const void* k, const void* v, void* o,

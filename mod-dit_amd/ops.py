@@ -79,6 +79,17 @@ class TileList:
         return (bits * valid).sum(dim=(1, 2))
 
 
+def _workspace(nbytes: int, device):
+    """(buffer, size) for a launch that can use `nbytes` of scratch: its own for each call, on
+    the current stream. Where the memory is not to be had, the launch runs without."""
+    if nbytes <= 0:
+        return None, 0
+    try:
+        return torch.empty(nbytes, device=device, dtype=torch.uint8), nbytes
+    except torch.cuda.OutOfMemoryError:
+        return None, 0
+
+
 def _attention(q, k, v, scale, return_lse, tiles: TileList | None, out=None):
     _require_gpu(q, k, v, what="attention")
     if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
@@ -107,10 +118,15 @@ def _attention(q, k, v, scale, return_lse, tiles: TileList | None, out=None):
             strides3(*q.stride()[:3]), strides3(*k.stride()[:3]), strides3(*v.stride()[:3]),
             strides3(*out.stride()[:3]), float(scale), dt)
     if tiles is None:
-        check(lib.moddit_flash_fwd(*args, _stream(q)), "moddit_flash_fwd")
+        ws, nbytes = _workspace(lib.moddit_flash_fwd_workspace_bytes(B, H, Sq, Skv, D), q.device)
+        check(lib.moddit_flash_fwd_ws(*args, _ptr(ws), nbytes, _stream(q)), "moddit_flash_fwd")
     else:
-        check(lib.moddit_block_sparse_fwd(*args, tiles.counts.data_ptr(), tiles.entries.data_ptr(),
-                                          tiles.n_qtiles, tiles.cap, int(tiles.origin), _stream(q)),
+        ws, nbytes = _workspace(
+            lib.moddit_block_sparse_fwd_workspace_bytes(B, H, Sq, D, tiles.cap, int(tiles.origin)),
+            q.device)
+        check(lib.moddit_block_sparse_fwd_ws(*args, tiles.counts.data_ptr(),
+                                             tiles.entries.data_ptr(), tiles.n_qtiles, tiles.cap,
+                                             int(tiles.origin), _ptr(ws), nbytes, _stream(q)),
               "moddit_block_sparse_fwd")
     return out, lse
 
