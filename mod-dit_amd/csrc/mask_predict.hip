@@ -120,187 +120,327 @@ __global__ __launch_bounds__(kMtsThreads) void mts_kernel(MtsParams p) {
 }
 
 // -------------------------------------------------------------------------------------
-// Single pass over an fp16 map (the product path). One workgroup per (head, 512-row x
-// 256-column tile) reads its cells once with 16-byte loads. Each thread owns 8 consecutive
-// columns of one 64-row slab of the tile and keeps its column sums and, per 16-row
-// sub-block, the sums of the 23 diagonals its 8 x 16 cells lie on in fp64 registers.
-// Every finite fp16 value is a multiple of 2^-24 below 2^16, so any sum of at most 8192 of
-// them needs at most 53 significant bits and is exact in fp64 in any order; a tile's
-// share of one line is at most 512 cells. The eight slabs' column sums and the threads'
-// overlapping diagonal sums are combined in LDS (still exact), and each workgroup adds
-// its column, diagonal and frame-block partials into an int64 accumulator per output
-// (units of 2^-24) with global integer atomics: exact and order-independent, so every
-// output is the correctly rounded fp32 of the exact sum in any workgroup order
-// (deterministic), and the map is read once (155.5 MB at the headline). A partial that is
-// not finite (inf/NaN inputs) goes into a float side accumulator instead (inf/NaN
-// semantics only, also order-independent). The tile shape minimises the global atomics
-// per cell for its area (256 column + 767 diagonal partials per 131,072 cells): contended
-// atomics, not the loads, were what bounded the 64-row-block version of this pass.
-constexpr int kMts1Threads = 256;
-constexpr int kMts1Cols = 8;         // columns per thread
-constexpr int kMts1Sub = 16;         // rows per register sub-block
-constexpr int kMts1Slab = 64;        // rows per thread
-constexpr int kMts1ColThreads = 32;  // threads across a tile's columns
-constexpr int kMts1Slabs = kMts1Threads / kMts1ColThreads;   // 8
-constexpr int kMts1TileC = kMts1ColThreads * kMts1Cols;      // 256
-constexpr int kMts1TileR = kMts1Slabs * kMts1Slab;           // 512
-constexpr int kMts1Diag = kMts1Cols + kMts1Sub - 1;          // 23
-constexpr int kMts1TileDiag = kMts1TileC + kMts1TileR - 1;   // 767
-// Exactness of the int64 accumulators: an fp16 value is below 2^16, i.e. 2^40 units of
-// 2^-24, so a sum over c cells stays below 2^63 while c <= 2^23. Diagonal and column
-// outputs sum n cells; the frame-block output sums (n / bpf) * bpf^2 = n * min(bpf, n)
-// cells, which the entry point bounds (kMts1MaxFrameCells).
+// Single pass over an fp16 map (the product path): mts_tile_kernel reads every cell once and
+// leaves one record of partial sums per tile, mts_sum_kernel adds the records of each line.
+//
+// A tile is 512 columns x 4R rows; each of the workgroup's four waves owns R rows, a lane 8
+// consecutive columns. Column sums stay in the lane. A diagonal moves one column to the
+// right per row, so the lane's 8 diagonal sums do too: their registers are renamed (the row
+// loop is unrolled by 8), the one that crosses to the next lane moves by a wave shift, and
+// the one that leaves the last lane is stored to LDS. Nothing is reduced across lanes, and
+// no atomic is used: with 23 LDS atomics per 8 x 16 cells and global atomics per tile, which
+// this replaced, the map took 62 us at n = 1800 x 24 (155.5 MB) and, where rows are not
+// 16-byte aligned, 85 us at n = 275 x 48 (7 MB, 96 workgroups), plus 9 us of clearing and
+// finishing launches; now 47.5 (3.3 TB/s) and 12 us, plus 7.3 and 4.7 us for the sums. It
+// issues 41 VALU instructions per row of 64 x 8 cells, half of them fp64, on three waves
+// per SIMD (148 VGPRs; held to 128 it spills and takes 89 us); a second register stage of
+// loads gains nothing.
+//
+// Exactness: every finite fp16 value is a multiple of 2^-24 below 2^16, so any sum of at
+// most 8192 of them needs at most 53 significant bits and is exact in fp64 in any order; a
+// tile's share of one line is at most 4R <= 256 cells. The records are then added as int64
+// in units of 2^-24 and rounded once to fp32: every output is the correctly rounded sum,
+// whatever the tile shape. Records that are not finite (inf/NaN inputs) are added in float
+// instead, in a fixed order (inf/NaN semantics only).
+constexpr int kMtsTileThreads = 256;
+constexpr int kMtsWaves = kMtsTileThreads / 64;
+constexpr int kMtsCols = 8;                    // columns per lane
+constexpr int kMtsTileC = 64 * kMtsCols;       // 512
+// Rows per wave: 64, or 16 for maps too small to fill the GPU with the taller tiles.
+constexpr int kMtsRowsTall = 64;
+constexpr int kMtsRowsShort = 16;
+constexpr int64_t kMtsFillTiles = 512;         // two workgroups per CU
+// A map's line sums over c cells stay below 2^63 units of 2^-24 while c <= 2^23 (an fp16
+// value is below 2^40 units). Diagonal and column outputs sum n cells; the frame-block
+// output sums (n / bpf) * bpf^2 = n * min(bpf, n) cells, which the entry point bounds.
 constexpr int kMts1MaxN = 1 << 20;
 constexpr int64_t kMts1MaxFrameCells = int64_t{1} << 23;
+
+// Record of a tile: its diagonals' sums (index kl = (c - C0) - (r - R0) + rows - 1), its
+// columns' sums, the frame-block sum in int64 units and its non-finite part.
+__host__ __device__ constexpr int mts_tile_diags(int rows) { return kMtsTileC + kMtsWaves * rows - 1; }
+__host__ __device__ constexpr int mts_record_doubles(int rows) { return mts_tile_diags(rows) + kMtsTileC + 2; }
+
+inline int mts_rows_for(int heads, int n) {
+  const int64_t ct = (n + kMtsTileC - 1) / kMtsTileC;
+  const int tall = kMtsWaves * kMtsRowsTall;
+  return heads * ct * ((n + tall - 1) / tall) >= kMtsFillTiles ? kMtsRowsTall : kMtsRowsShort;
+}
 
 struct Mts1Params {
   const uint16_t* map;
   int heads;
   int n;
   int bpf;
-  int n_rt;  // row tiles per head
-  int n_ct;  // column tiles per head
-  unsigned long long* acc;  // (H, 3n) int64 units of 2^-24 (two's complement)
-  float* special;           // (H, 3n) sums of the non-finite partials
-  float* out;               // (H, 3n)
+  int n_rt;        // row tiles per head
+  int n_ct;        // column tiles per head
+  double* records; // [head][row tile][column tile][mts_record_doubles(rows)]
+  float* out;      // (H, 3n)
 };
 
-// Adds an exact fp64 partial (a multiple of 2^-24, |x| < 2^25) to an output.
-__device__ __forceinline__ void mts1_flush(const Mts1Params& p, int64_t idx, double x) {
-  if (x == 0.0) return;
-  if (__builtin_isfinite(x)) {
-    atomicAdd(&p.acc[idx], static_cast<unsigned long long>(static_cast<long long>(x * 0x1p24)));
-  } else {
-    atomicAdd(&p.special[idx], static_cast<float>(x));
-  }
+// x of the previous lane (0 in lane 0)
+__device__ __forceinline__ double wave_shift_up(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(u), 0x138, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(u >> 32), 0x138, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, static_cast<uint64_t>(lo) | (static_cast<uint64_t>(hi) << 32));
 }
 
-__global__ void mts1_zero_kernel(Mts1Params p) {
-  const int64_t total = static_cast<int64_t>(p.heads) * 3 * p.n;
-  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    p.acc[i] = 0ull;
-    p.special[i] = 0.f;
-  }
+__device__ __forceinline__ double read_lane(double x, int lane) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(u), lane);
+  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(u >> 32), lane);
+  return __builtin_bit_cast(double, static_cast<uint64_t>(lo) | (static_cast<uint64_t>(hi) << 32));
 }
 
-template <bool kVec>
-__global__ __launch_bounds__(kMts1Threads) void mts1_kernel(Mts1Params p) {
-  __shared__ double s_diag[kMts1TileDiag];
-  __shared__ double s_col[kMts1Slabs][kMts1TileC];
-  __shared__ long long s_frame[kMts1Threads / 64];
+template <int kRows>
+__global__ __launch_bounds__(kMtsTileThreads, 3) void mts_tile_kernel(Mts1Params p) {
+  constexpr int kWaveDiag = kMtsTileC + kRows - 1;
+  constexpr int kTileDiag = mts_tile_diags(kRows);
+  __shared__ double s_diag[kMtsWaves][kWaveDiag];
+  __shared__ double s_col[kMtsWaves][kMtsTileC];
+  __shared__ long long s_frame[kMtsWaves];
+  __shared__ double s_special[kMtsWaves];
   const int tid = threadIdx.x;
-  const int tc = tid % kMts1ColThreads;
-  const int tr = tid / kMts1ColThreads;
+  const int lane = tid & 63;
+  // wave-uniform, so that the row tests and addresses below are scalar
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = p.n;
   const int tiles = p.n_rt * p.n_ct;
   const int h = blockIdx.x / tiles;
   const int t = blockIdx.x - h * tiles;
-  const int R0 = (t / p.n_ct) * kMts1TileR;
-  const int C0 = (t % p.n_ct) * kMts1TileC;
-  const int n = p.n;
-  const int nd = 2 * n - 1;
-  const int64_t F = 3 * static_cast<int64_t>(n);
+  const int R0 = (t / p.n_ct) * (kMtsWaves * kRows);
+  const int C0 = (t % p.n_ct) * kMtsTileC;
+  const int rs = R0 + wave * kRows;        // this wave's first row
+  const int c0 = C0 + lane * kMtsCols;     // this lane's first column
+  const int64_t cells = static_cast<int64_t>(p.heads) * n * n;
+  const int64_t head0 = static_cast<int64_t>(h) * n * n;
   const int frame_end = (n / p.bpf) * p.bpf;
-  for (int i = tid; i < kMts1TileDiag; i += kMts1Threads) s_diag[i] = 0.0;
-  __syncthreads();
+  // columns past the row's end are loaded with the next row's cells and cleared
+  u32x4 keep;
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+    keep[w] = (c0 + 2 * w < n ? 0xffffu : 0u) | (c0 + 2 * w + 1 < n ? 0xffff0000u : 0u);
 
-  const int c0 = C0 + tc * kMts1Cols;   // this thread's first column
-  const int rs = R0 + tr * kMts1Slab;   // this thread's first row
-  const uint16_t* base = p.map + static_cast<int64_t>(h) * n * n;
-  const int64_t out0 = static_cast<int64_t>(h) * F;
-  // frames of the first and last owned columns inside the frame blocks (-1: none)
-  const int c_last = (c0 + kMts1Cols - 1 < frame_end ? c0 + kMts1Cols - 1 : frame_end - 1);
-  const int cf_lo = c0 < frame_end ? c0 / p.bpf : -1;
-  const int cf_hi = c0 < frame_end ? c_last / p.bpf : -1;
-  double cacc[kMts1Cols];
+  double cacc[kMtsCols], dacc[kMtsCols];
 #pragma unroll
-  for (int j = 0; j < kMts1Cols; ++j) cacc[j] = 0.0;
+  for (int j = 0; j < kMtsCols; ++j) cacc[j] = dacc[j] = 0.0;
   double fsum = 0.0;
-  if (c0 < n) {
-    for (int s0 = 0; s0 < kMts1Slab; s0 += kMts1Sub) {
-      if (rs + s0 >= n) break;
-      double dacc[kMts1Diag];
+  double leaving = 0.0;  // lane i: the diagonal that left the last lane after row i
+  // the cells of one row, with the lane's diagonal of column j in register (j - rr) & 7
+  auto add_row = [&](u32x4 w, int rr) {
 #pragma unroll
-      for (int d = 0; d < kMts1Diag; ++d) dacc[d] = 0.0;
+    for (int j = 0; j < kMtsCols; ++j) {
+      const double x = static_cast<double>(Fp16::to_float(u16_at(w, j)));
+      cacc[j] += x;
+      dacc[(j - rr) & 7] += x;
+    }
+  };
+  // its frame-block cells, if the row's frame meets the tile's columns
+  auto add_frame = [&](u32x4 w, int r) {
+    const int f0 = r < frame_end ? r / p.bpf * p.bpf : n;
+    if (f0 < C0 + kMtsTileC && f0 + p.bpf > C0) {
 #pragma unroll
-      for (int rr = 0; rr < kMts1Sub; ++rr) {
-        const int r = rs + s0 + rr;
-        if (r < n) {
-          const uint16_t* row = base + static_cast<int64_t>(r) * n;
-          uint16_t v[kMts1Cols];
-          if constexpr (kVec) {
-            const u32x4 w = *reinterpret_cast<const u32x4*>(row + c0);
+      for (int j = 0; j < kMtsCols; ++j)
+        if (static_cast<unsigned>(c0 + j - f0) < static_cast<unsigned>(p.bpf))
+          fsum += static_cast<double>(Fp16::to_float(u16_at(w, j)));
+    }
+  };
+  // one row down, the diagonals are one column further: the sum at column 7 goes to the next
+  // lane, the last lane's is complete
+  auto step_down = [&](double& edge, int row) {
+    const double out = read_lane(edge, 63);
+    leaving = lane == row ? out : leaving;
+    edge = wave_shift_up(edge);
+  };
+#pragma unroll 1
+  for (int r8 = 0; r8 < kRows; r8 += 8) {
+    const int r = rs + r8;
+    if (r + 8 <= n && head0 + static_cast<int64_t>(r + 7) * n + C0 + kMtsTileC <= cells) {
+      // eight whole rows, 16 bytes per lane at any 2-byte address
+      u32x4 raw[8];
+      const uint16_t* src = p.map + head0 + static_cast<int64_t>(r) * n + (c0 < n ? c0 : C0);
 #pragma unroll
-            for (int j = 0; j < kMts1Cols; ++j) v[j] = u16_at(w, j);
-          } else {
+      for (int rr = 0; rr < 8; ++rr) __builtin_memcpy(&raw[rr], src + static_cast<int64_t>(rr) * n, 16);
 #pragma unroll
-            for (int j = 0; j < kMts1Cols; ++j) v[j] = c0 + j < n ? row[c0 + j] : 0;
-          }
-          double x[kMts1Cols];
-#pragma unroll
-          for (int j = 0; j < kMts1Cols; ++j) {
-            x[j] = static_cast<double>(Fp16::to_float(v[j]));
-            cacc[j] += x[j];
-            dacc[j - rr + kMts1Sub - 1] += x[j];
-          }
-          // frame-block cells: only rows whose frame meets the owned columns
-          const int rframe = r < frame_end ? r / p.bpf : -2;
-          if (rframe >= cf_lo && rframe <= cf_hi) {
-#pragma unroll
-            for (int j = 0; j < kMts1Cols; ++j)
-              if (c0 + j < frame_end && (c0 + j) / p.bpf == rframe) fsum += x[j];
-          }
-        }
+      for (int rr = 0; rr < 8; ++rr) {
+        raw[rr] &= keep;
+        add_row(raw[rr], rr);
+        step_down(dacc[(7 - rr) & 7], r8 + rr);
+        __builtin_amdgcn_sched_barrier(0);  // or all 64 cells are converted first, and spill
       }
-      // local diagonal kl = (c - C0) - (r - R0) + 511 of accumulator d
+      // The frame cells apart from the sums above, which stay free of branches. The empty asm
+      // keeps the compiler from moving the sums below these branches, and from carrying the
+      // 64 converted cells across them: either spills.
 #pragma unroll
-      for (int d = 0; d < kMts1Diag; ++d) {
-        const int kl = (c0 - C0) + d - (kMts1Sub - 1) - (rs - R0) - s0 + (kMts1TileR - 1);
-        if (dacc[d] != 0.0) atomicAdd(&s_diag[kl], dacc[d]);
+      for (int j = 0; j < kMtsCols; ++j) asm volatile("" : "+v"(cacc[j]), "+v"(dacc[j]));
+#pragma unroll
+      for (int rr = 0; rr < 8; ++rr) {
+        asm volatile("" : "+v"(raw[rr]));
+        add_frame(raw[rr], r + rr);
+      }
+    } else {
+      // the last rows, cell by cell: nothing past the map's end is touched
+#pragma unroll 1
+      for (int rr = 0; rr < 8; ++rr) {
+        uint64_t lo = 0, hi = 0;
+        const uint16_t* src = p.map + head0 + static_cast<int64_t>(r + rr) * n + c0;
+        const int m = r + rr < n ? (n - c0 < kMtsCols ? n - c0 : kMtsCols) : 0;
+#pragma unroll 1
+        for (int j = 0; j < m; ++j) {
+          const uint64_t v = src[j];
+          if (j < 4)
+            lo |= v << (16 * j);
+          else
+            hi |= v << (16 * (j - 4));
+        }
+        const u32x4 raw = {static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32),
+                           static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32)};
+        add_row(raw, 0);
+        add_frame(raw, r + rr);
+        step_down(dacc[7], r8 + rr);
+        const double edge = dacc[7];
+#pragma unroll
+        for (int j = kMtsCols - 1; j > 0; --j) dacc[j] = dacc[j - 1];
+        dacc[0] = edge;
       }
     }
   }
+  // after the last row's shift, register j of lane l holds the diagonal of column 8l + j - 1
 #pragma unroll
-  for (int j = 0; j < kMts1Cols; ++j) s_col[tr][tc * kMts1Cols + j] = cacc[j];
-  // frame-block partial of the workgroup: each thread's sum (at most 512 cells) is exact in
-  // fp64 and converts exactly to int64 units; the workgroup adds them as integers
+  for (int j = 0; j < kMtsCols; ++j) {
+    const int kl = lane * kMtsCols + j - 1;
+    if (kl >= 0) s_diag[wave][kl] = dacc[j];
+    s_col[wave][lane * kMtsCols + j] = cacc[j];
+  }
+  if (lane < kRows) s_diag[wave][kWaveDiag - 1 - lane] = leaving;
+  // frame-block partial: each lane's sum (at most 512 cells) is exact in fp64 and converts
+  // exactly to int64 units
   long long fq = 0;
+  double special = 0.0;
   if (__builtin_isfinite(fsum))
     fq = static_cast<long long>(fsum * 0x1p24);
   else
-    atomicAdd(&p.special[out0 + F - 1], static_cast<float>(fsum));
+    special = fsum;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) fq += __shfl_xor(fq, o);
-  if ((tid & 63) == 0) s_frame[tid >> 6] = fq;
-  __syncthreads();
-  if (tid == 0) {
-    long long tot = 0;
-    for (int w = 0; w < kMts1Threads / 64; ++w) tot += s_frame[w];
-    if (tot != 0) atomicAdd(&p.acc[out0 + F - 1], static_cast<unsigned long long>(tot));
+  for (int o = 32; o > 0; o >>= 1) {
+    fq += __shfl_xor(fq, o);
+    special += __shfl_xor(special, o);
   }
-  // column partials: the eight slabs' sums of one column (at most 512 cells, exact)
-  for (int c = tid; c < kMts1TileC; c += kMts1Threads) {
+  if (lane == 0) {
+    s_frame[wave] = fq;
+    s_special[wave] = special;
+  }
+  __syncthreads();
+
+  double* rec = p.records + static_cast<int64_t>(blockIdx.x) * mts_record_doubles(kRows);
+  // wave w's index is kl minus the rows below it in the tile
+  for (int kl = tid; kl < kTileDiag; kl += kMtsTileThreads) {
     double sum = 0.0;
 #pragma unroll
-    for (int sl = 0; sl < kMts1Slabs; ++sl) sum += s_col[sl][c];
-    if (C0 + c < n) mts1_flush(p, out0 + nd + C0 + c, sum);
+    for (int w = 0; w < kMtsWaves; ++w) {
+      const int i = kl - (kMtsWaves - 1 - w) * kRows;
+      if (i >= 0 && i < kWaveDiag) sum += s_diag[w][i];
+    }
+    rec[kl] = sum;
   }
-  // diagonal partials: global index k = (c - r) + n - 1 = kl - 511 + C0 - R0 + n - 1
-  for (int kl = tid; kl < kMts1TileDiag; kl += kMts1Threads) {
-    const int k = kl - (kMts1TileR - 1) + C0 - R0 + n - 1;
-    if (k >= 0 && k < nd) mts1_flush(p, out0 + k, s_diag[kl]);
+  for (int c = tid; c < kMtsTileC; c += kMtsTileThreads)
+    rec[kTileDiag + c] = (s_col[0][c] + s_col[1][c]) + (s_col[2][c] + s_col[3][c]);
+  if (tid == 0) {
+    rec[kTileDiag + kMtsTileC] =
+        __builtin_bit_cast(double, (s_frame[0] + s_frame[1]) + (s_frame[2] + s_frame[3]));
+    rec[kTileDiag + kMtsTileC + 1] = (s_special[0] + s_special[1]) + (s_special[2] + s_special[3]);
   }
 }
 
-__global__ void mts1_finalize_kernel(Mts1Params p) {
-  const int64_t total = static_cast<int64_t>(p.heads) * 3 * p.n;
-  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-    const float sp = p.special[i];
-    p.out[i] = (sp != 0.f || sp != sp)
-                   ? sp
-                   : static_cast<float>(static_cast<long long>(p.acc[i])) * 0x1p-24f;
+// Exact sum of finite fp64 partials (multiples of 2^-24); non-finite ones apart, in float.
+struct MtsSum {
+  long long q = 0;
+  float special = 0.f;
+  __device__ __forceinline__ void add(double x) {
+    if (__builtin_isfinite(x))
+      q += static_cast<long long>(x * 0x1p24);
+    else
+      special += static_cast<float>(x);
   }
+  __device__ __forceinline__ float result() const {
+    return (special != 0.f || special != special) ? special : static_cast<float>(q) * 0x1p-24f;
+  }
+};
+
+// One thread per diagonal and column output, one wave per head's frame-block output.
+template <int kRows>
+__global__ __launch_bounds__(kMtsTileThreads) void mts_sum_kernel(Mts1Params p) {
+  constexpr int kTileR = kMtsWaves * kRows;
+  constexpr int kTileDiag = mts_tile_diags(kRows);
+  constexpr int kRec = mts_record_doubles(kRows);
+  const int n = p.n;
+  const int nd = 2 * n - 1;
+  const int64_t F = 3 * static_cast<int64_t>(n);
+  const int groups = static_cast<int>((F - 1 + kMtsTileThreads - 1) / kMtsTileThreads) + 1;
+  const int h = blockIdx.x / groups;
+  const int g = blockIdx.x - h * groups;
+  const double* rec = p.records + static_cast<int64_t>(h) * p.n_rt * p.n_ct * kRec;
+  float* out = p.out + static_cast<int64_t>(h) * F;
+  if (g == groups - 1) {  // frame blocks: lanes stride the tiles
+    if (threadIdx.x >= 64) return;
+    long long q = 0;
+    double special = 0.0;
+    for (int64_t t = threadIdx.x; t < static_cast<int64_t>(p.n_rt) * p.n_ct; t += 64) {
+      q += __builtin_bit_cast(long long, rec[t * kRec + kTileDiag + kMtsTileC]);
+      special += rec[t * kRec + kTileDiag + kMtsTileC + 1];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      q += __shfl_xor(q, o);
+      special += __shfl_xor(special, o);
+    }
+    if (threadIdx.x == 0) {
+      MtsSum sum;
+      sum.q = q;
+      sum.special = static_cast<float>(special);
+      out[F - 1] = sum.result();
+    }
+    return;
+  }
+  const int64_t i = static_cast<int64_t>(g) * kMtsTileThreads + threadIdx.x;
+  if (i >= F - 1) return;
+  MtsSum sum;
+  if (i < nd) {
+    // diagonal offset c - r = off crosses row tile rt at columns [R0 + off, R0 + off + kTileR)
+    const int off = static_cast<int>(i) - (n - 1);
+    for (int rt = 0; rt < p.n_rt; ++rt) {
+      const int first = rt * kTileR + off;
+      const int last = first + kTileR - 1;
+      if (last < 0 || first >= n) continue;
+      const int ct0 = (first < 0 ? 0 : first) / kMtsTileC;
+      const int ct1 = (last < n ? last : n - 1) / kMtsTileC;
+      for (int ct = ct0; ct <= ct1; ++ct)
+        sum.add(rec[(static_cast<int64_t>(rt) * p.n_ct + ct) * kRec + first - ct * kMtsTileC + kTileR - 1]);
+    }
+  } else {
+    const int c = static_cast<int>(i) - nd;
+    for (int rt = 0; rt < p.n_rt; ++rt)
+      sum.add(rec[(static_cast<int64_t>(rt) * p.n_ct + c / kMtsTileC) * kRec + kTileDiag + c % kMtsTileC]);
+  }
+  out[i] = sum.result();
+}
+
+template <int kRows>
+int launch_mts_fp16(Mts1Params& q, hipStream_t st) {
+  q.n_rt = (q.n + kMtsWaves * kRows - 1) / (kMtsWaves * kRows);
+  q.n_ct = (q.n + kMtsTileC - 1) / kMtsTileC;
+  const int64_t grid = static_cast<int64_t>(q.heads) * q.n_rt * q.n_ct;
+  const int64_t sums = static_cast<int64_t>(q.heads) *
+                       ((3 * static_cast<int64_t>(q.n) - 1 + kMtsTileThreads - 1) / kMtsTileThreads + 1);
+  MODDIT_CHECK_ARG(grid < 0x7fffffff && sums < 0x7fffffff, "mts: shape too large");
+  hipLaunchKernelGGL((mts_tile_kernel<kRows>), dim3(static_cast<unsigned>(grid)),
+                     dim3(kMtsTileThreads), 0, st, q);
+  MODDIT_CHECK_LAUNCH("mts");
+  hipLaunchKernelGGL((mts_sum_kernel<kRows>), dim3(static_cast<unsigned>(sums)),
+                     dim3(kMtsTileThreads), 0, st, q);
+  MODDIT_CHECK_LAUNCH("mts (sum)");
+  return MODDIT_OK;
 }
 
 // =====================================================================================
@@ -743,7 +883,10 @@ using namespace moddit;
 
 extern "C" int64_t moddit_mts_workspace_bytes(int heads, int n) {
   if (heads <= 0 || n <= 0) return 0;
-  return static_cast<int64_t>(heads) * 3 * n * (sizeof(unsigned long long) + sizeof(float));
+  const int rows = mts_rows_for(heads, n);
+  const int64_t n_rt = (n + kMtsWaves * rows - 1) / (kMtsWaves * rows);
+  const int64_t n_ct = (n + kMtsTileC - 1) / kMtsTileC;
+  return heads * n_rt * n_ct * mts_record_doubles(rows) * static_cast<int64_t>(sizeof(double));
 }
 
 extern "C" int moddit_mts(const void* map, int map_dtype, int heads, int n, int blocks_per_frame,
@@ -773,25 +916,10 @@ extern "C" int moddit_mts(const void* map, int map_dtype, int heads, int n, int 
     q.heads = heads;
     q.n = n;
     q.bpf = blocks_per_frame;
-    q.n_rt = (n + kMts1TileR - 1) / kMts1TileR;
-    q.n_ct = (n + kMts1TileC - 1) / kMts1TileC;
-    const int64_t total = static_cast<int64_t>(heads) * 3 * n;
-    q.acc = static_cast<unsigned long long*>(workspace);
-    q.special = reinterpret_cast<float*>(q.acc + total);
+    q.records = static_cast<double*>(workspace);
     q.out = mts_out;
-    const int64_t grid = static_cast<int64_t>(heads) * q.n_rt * q.n_ct;
-    MODDIT_CHECK_ARG(grid < 0x7fffffff, "mts: shape too large");
-    int64_t fill = (total + 255) / 256;
-    if (fill > 4096) fill = 4096;
-    hipLaunchKernelGGL(mts1_zero_kernel, dim3(static_cast<unsigned>(fill)), dim3(256), 0, st, q);
-    MODDIT_CHECK_LAUNCH("mts (zero)");
-    const bool vec = n % 8 == 0 && aligned16(map);
-    auto kernel = vec ? mts1_kernel<true> : mts1_kernel<false>;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kMts1Threads), 0, st, q);
-    MODDIT_CHECK_LAUNCH("mts");
-    hipLaunchKernelGGL(mts1_finalize_kernel, dim3(static_cast<unsigned>(fill)), dim3(256), 0, st, q);
-    MODDIT_CHECK_LAUNCH("mts (finalize)");
-    return MODDIT_OK;
+    return mts_rows_for(heads, n) == kMtsRowsTall ? launch_mts_fp16<kMtsRowsTall>(q, st)
+                                                  : launch_mts_fp16<kMtsRowsShort>(q, st);
   }
   MtsParams p;
   p.map = static_cast<const float*>(map);
