@@ -111,5 +111,8 @@ def check(rc: int, what: str) -> None:
         raise ModditError(f"{what} failed (status {rc}): {msg}")
 
 
+_i64x3 = ctypes.c_int64 * 3
+
+
 def strides3(*vals: int):
-    return (ctypes.c_int64 * 3)(*vals)
+    return _i64x3(*vals)

@@ -1,20 +1,31 @@
 // Dense and block-sparse flash-attention forward for gfx950 (CDNA4).
 //
-// One workgroup = 4 wave64s = 128 query rows (each wave owns 32 rows); keys stream in
-// tiles of 64 (the mask's key-block granularity). Per key tile each wave computes
-//   S^T (64 keys x 32 queries) = K . Q^T      with 2 x 8 (d=128) bf16 MFMA 32x32x16
-//   O^T (d x 32 queries)      += V^T . P^T    with (d/32) x 4 MFMA 32x32x16
-// Computing the transposed products puts one query per lane column, so the running
-// row max / row sum live in one lane (plus one exchange with the lane 32 apart) and
-// the rescale of O is a per-lane multiply. The S^T accumulator layout is exactly the
-// B-operand layout P^T needs, so P never leaves registers.
+// One workgroup = 4 wave64s = 128 query rows (each wave owns 32 rows as two 16-row blocks);
+// keys stream in tiles of 64 (the mask's key-block granularity). Per key tile each wave
+// computes, on bf16/fp16 MFMA 16x16x32,
+//   S^T (64 keys x 32 queries) = K . Q^T      4 key x 2 query blocks, D/32 steps
+//   O^T (d x 32 queries)      += V^T . P^T    D/16 x 2 blocks, 2 steps
+// Computing the transposed products puts one query per lane column and block, so the rescale
+// of O is a per-lane multiply, and the S^T accumulators of key blocks 2t and 2t+1 are the
+// B operand of P^T's step t (the V operand is read in the same key order), so P never
+// leaves registers.
+//
+// What bounds it is the board's power limit: the clock falls until the power fits, so time
+// follows the energy of the work, not its schedule. The 16x16x32 shape does the same
+// products for less (2.19 against 1.86 PFLOP/s for 32x32x16 on random operands at the
+// limit). Its price, two queries per lane and with them twice the row reductions, is not
+// paid on most tiles: the softmax takes the running max as it is and checks the lane's sum
+// of weights afterwards (softmax_kept). Against the 32x32x16 kernel with a max per tile, on
+// structured inputs: dense 24 heads x 115,200, D = 128 145.9 -> 137.2 ms (1,190 TFLOP/s; a
+// hipBLASLt GEMM of 8,192^3 runs at 1,180 there), block-sparse 40 x 69,120 20.0 -> 19.0 ms,
+// 48 x 17,776, D = 64 1.45 -> 1.41 ms.
 //
 // K and V tiles go straight from HBM into LDS (buffer_load ... lds, no register
 // staging), both row-major with an XOR swizzle on 16-byte chunks that keeps the operand
 // reads bank-conflict free; V^T fragments come out of the row-major V tile through
 // ds_read_b64_tr_b16. Two stages per operand. The loop is software pipelined:
-// iteration j computes S_{j+1} and O += P_j V_j while K_{j+2} and V_{j+1} stream in, then
-// the softmax of S_{j+1}; one barrier per tile.
+// iteration j computes S_{j+1}, then O += P_j V_j together with the softmax of S_{j+1}, while
+// K_{j+2} and V_{j+1} stream in; one barrier per tile.
 //
 // The sparse variant walks a per-(head, query tile) list of key tiles, each entry
 // carrying two row bits (query rows 0-63 / 64-127 of the tile); a wave whose bit is
@@ -82,23 +93,25 @@ struct AttnParams {
   float* part_ml;  // [tile][piece][128][2]: running max (log2 units) and row sum
 };
 
-// K rows are stored in LDS in the order pi(r): inside every 16-row chunk the row groups
-// [4,8) and [8,12) are swapped, so the S^T accumulator of lane half h holds keys
-// 8h..8h+7 of each 16-key chunk, in order (the P^T operand needs no shuffle).
-__device__ __forceinline__ int key_perm(int r) { return r ^ ((((r >> 2) ^ (r >> 3)) & 1) * 12); }
-
 // 16-byte chunk swizzles (XOR on the chunk index) that make the MFMA operand reads
 // bank-conflict free: K rows are read one row per lane (A operand of S^T), V rows
-// through ds_read_b64_tr_b16 (four keys x 32 dims per half-wave).
+// through ds_read_b64_tr_b16 (eight keys x 16 dims per half-wave).
 template <int D>
 __device__ __forceinline__ int swz_k(int r) { return (r / (128 / D)) % (D / 8); }
 template <int D>
-__device__ __forceinline__ int swz_v(int key) { return 4 * ((key / (128 / D)) % (D / 32)); }
+__device__ __forceinline__ int swz_v(int key) { return 2 * ((key / (128 / D)) % (D / 16)); }
 
-// The running row max is only moved when a tile's max exceeds it by more than this many
-// log2 units; probabilities then stay <= 2^8 and the O rescale is skipped for whole
-// waves on most tiles. Softmax is shift-invariant, so results do not depend on it.
+// The running row max is not looked at on most tiles: a tile's weights are taken against the
+// max as it is, and only if a lane's sum of them reaches kMaxWeightSum does the tile go
+// through the general softmax, which then moves every row's max to the tile's where that is
+// larger. On other tiles that take the general softmax (the first, boundaries, exact rows'
+// gaps) it moves by more than kRescaleSlack log2 units only. Softmax is shift-invariant, so
+// results do not depend on either, but for the rounding of P: a row's largest weight is
+// exact (1) where the max is its own. The limit 256 = 2^kRescaleSlack keeps the error
+// against fp64 at that of a max per tile (2.16e-3 and 2.17e-3 of the result on the
+// Wan-like layer); 1,024 and 2^20 are up to 1 and 2 % faster there, at 2.22e-3 and 2.31e-3.
 constexpr float kRescaleSlack = 8.0f;
+constexpr float kMaxWeightSum = 256.0f;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -119,8 +132,8 @@ template <int D, typename E, bool kSparse, bool kRagged, bool kMap = false, bool
 __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_fwd_kernel(AttnParams p) {
   using L = AttnLds<D>;
   using V8 = typename E::vec8;
-  constexpr int kDChunks = D / 16;  // MFMA k-steps over d for S^T
-  constexpr int kDSub = D / 32;     // 32-row blocks of O^T
+  constexpr int kKC = D / 32;  // MFMA k-steps over d for S^T
+  constexpr int kDB = D / 16;  // 16-row blocks of O^T
   constexpr int kWinPerWave = L::kWindows / 4;
 
   extern __shared__ __align__(16) unsigned char smem[];
@@ -130,8 +143,8 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   const int tid = threadIdx.x;
   const int wave = tid >> 6;
   const int lane = tid & 63;
-  const int half = lane >> 5;
-  const int c32 = lane & 31;
+  const int g = lane >> 4;
+  const int c16 = lane & 15;
 
   const int tile = kSplit ? blockIdx.x / p.n_split : xcd_remap(blockIdx.x, gridDim.x, p.xcd_run);
   const int qt = tile % p.n_qtiles;
@@ -165,17 +178,19 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   }
   const int wbit = 1 << (wave >> 1);
 
-  // ---- Q fragments (B operand of S^T = K Q^T): lane holds query c32, dims 8*half.. ----
+  // ---- Q fragments (B operand of S^T = K Q^T): lane holds query 16qq + c16, dims 32c + 8g.. ----
   // Grid rows outside [0, q_len) are padding: they load a clamped row and store nothing.
-  const int q_row = p.origin + qt * kBM + wave * 32 + c32;
-  V8 qf[kDChunks];
-  {
+  const int q_row0 = p.origin + qt * kBM + wave * 32 + c16;  // and + 16
+  V8 qf[2][kKC];
+#pragma unroll
+  for (int qq = 0; qq < 2; ++qq) {
+    const int q_row = q_row0 + 16 * qq;
     const int r = q_row < 0 ? 0 : (q_row < p.q_len ? q_row : p.q_len - 1);
     const u32x4* src = reinterpret_cast<const u32x4*>(qb + r * p.q_ss);
 #pragma unroll
-    for (int c = 0; c < kDChunks; ++c) qf[c] = as_vec8<V8>(src[2 * c + half]);
-    __builtin_amdgcn_s_waitcnt(0);
+    for (int c = 0; c < kKC; ++c) qf[qq][c] = as_vec8<V8>(src[4 * c + g]);
   }
+  __builtin_amdgcn_s_waitcnt(0);
 
   // ---- direct global -> LDS staging (buffer_load ... lds, 16 B per lane) ----
   // DMA window w writes LDS bytes [w*1024, w*1024+1024) of a stage, lane l at l*16. The
@@ -193,7 +208,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     const int pch = ((lane * 16) % L::kRowBytes) / 16;                  // physical chunk
     const int kq = pch ^ swz_k<D>(r);                                   // logical chunk
     const int vq = pch ^ swz_v<D>(r);
-    k_src[i] = static_cast<uint32_t>((key_perm(r) * p.k_ss + kq * 8) * 2);
+    k_src[i] = static_cast<uint32_t>((r * p.k_ss + kq * 8) * 2);
     v_src[i] = static_cast<uint32_t>((r * p.v_ss + vq * 8) * 2);
   }
   const uint32_t k_tile_bytes = static_cast<uint32_t>(kBN * p.k_ss * 2);
@@ -227,28 +242,29 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   };
 
   // ---- LDS operand addressing ----
-  // K (A operand of S^T): lane reads row c32 (+32), logical chunk 2c+half.
-  uint32_t k_rd[kDChunks];
+  // K (A operand of S^T): lane reads row 16kb + c16, logical chunk 4c + g.
+  uint32_t k_rd[kKC];
 #pragma unroll
-  for (int c = 0; c < kDChunks; ++c)
-    k_rd[c] = static_cast<uint32_t>(c32 * L::kRowBytes + (((2 * c + half) ^ swz_k<D>(c32)) * 16));
-  // V (A operand of O^T, via ds_read_b64_tr_b16): in 16-lane group g (dgrp = g&1,
-  // hh = g>>1) lane t addresses key 8*hh + (t>>2) (+16c + 4s) and dims dsub*32 + 16*dgrp + 4*(t&3).
-  const int g16 = lane >> 4;
-  const int t16 = lane & 15;
-  const int v_key0 = 8 * (g16 >> 1) + (t16 >> 2);  // key within a 16-key chunk, s = 0
-  uint32_t v_rd[kDSub];
+  for (int c = 0; c < kKC; ++c)
+    k_rd[c] = static_cast<uint32_t>(c16 * L::kRowBytes + (((4 * c + g) ^ swz_k<D>(c16)) * 16));
+  // V (A operand of O^T, via ds_read_b64_tr_b16): in 16-lane group g lane c16 addresses key
+  // 4g + c16/4 (+ 32t + 16s) and dims 16db + 4(c16%4).., and receives dim 16db + c16 of keys
+  // 32t + 16s + 4g .. +3. With s = 0 and 1 in the two halves of the operand, k index 8g + e
+  // is key 32t + 4g + e (e < 4) or 32t + 12 + 4g + e: the keys of the lane's own scores in
+  // key blocks 2t and 2t + 1, so P needs no shuffle.
+  const int v_key0 = 4 * g + (c16 >> 2);
+  uint32_t v_rd[kDB];
 #pragma unroll
-  for (int dsub = 0; dsub < kDSub; ++dsub) {
-    const int d = dsub * 32 + 16 * (g16 & 1) + 4 * (t16 & 3);
-    v_rd[dsub] = static_cast<uint32_t>(v_key0 * L::kRowBytes + (((d >> 3) ^ swz_v<D>(v_key0)) * 16) + (d & 7) * 2);
+  for (int db = 0; db < kDB; ++db) {
+    const int d = db * 16 + 4 * (c16 & 3);
+    v_rd[db] = static_cast<uint32_t>(v_key0 * L::kRowBytes + (((d >> 3) ^ swz_v<D>(v_key0)) * 16) + (d & 7) * 2);
   }
 
-  f32x16 oacc[kDSub];
+  f32x4 oacc[kDB][2];
 #pragma unroll
-  for (int i = 0; i < kDSub; ++i) oacc[i] = f32x16{};
-  float m_run = -INFINITY;
-  float l_run = 0.f;
+  for (int db = 0; db < kDB; ++db) oacc[db][0] = oacc[db][1] = f32x4{};
+  float m_run[2] = {-INFINITY, -INFINITY};
+  float l_run[2] = {0.f, 0.f};  // this lane's keys only
 
   auto decode = [&](int e_raw, int& kt, int& flags) {
     const int e = __builtin_amdgcn_readfirstlane(e_raw);
@@ -261,75 +277,112 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   };
   auto entry = [&](int i) -> int { return kSparse ? list[i] : (((it0 + i) << 2) | 3); };
 
-  auto qk = [&](const unsigned char* ks, f32x16& s0, f32x16& s1) {
-    s0 = f32x16{};
-    s1 = f32x16{};
+  // s[kb][qq][j]: key 16kb + 4g + j, query 16qq + c16
+  auto qk = [&](const unsigned char* ks, f32x4 (&s)[4][2]) {
 #pragma unroll
-    for (int c = 0; c < kDChunks; ++c) {
-      const V8 a0 = *reinterpret_cast<const V8*>(ks + k_rd[c]);
-      const V8 a1 = *reinterpret_cast<const V8*>(ks + k_rd[c] + 32 * L::kRowBytes);
-      s0 = E::mma(a0, qf[c], s0);
-      s1 = E::mma(a1, qf[c], s1);
-    }
-  };
-  auto pv = [&](const unsigned char* vs, const V8* pb) {
+    for (int kb = 0; kb < 4; ++kb) s[kb][0] = s[kb][1] = f32x4{};
 #pragma unroll
-    for (int dsub = 0; dsub < kDSub; ++dsub) {
+    for (int c = 0; c < kKC; ++c) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const unsigned char* a = vs + v_rd[dsub] + c * 16 * L::kRowBytes;
-        const s16x4 lo = lds_read_tr16(a);
-        const s16x4 hi = lds_read_tr16(a + 4 * L::kRowBytes);
-        const u32x4 w = {__builtin_bit_cast(u32x2, lo).x, __builtin_bit_cast(u32x2, lo).y,
-                         __builtin_bit_cast(u32x2, hi).x, __builtin_bit_cast(u32x2, hi).y};
-        oacc[dsub] = E::mma(as_vec8<V8>(w), pb[c], oacc[dsub]);
+      for (int kb = 0; kb < 4; ++kb) {
+        const V8 a = *reinterpret_cast<const V8*>(ks + k_rd[c] + 16 * kb * L::kRowBytes);
+        s[kb][0] = E::mma16(a, qf[0][c], s[kb][0]);
+        s[kb][1] = E::mma16(a, qf[1][c], s[kb][1]);
       }
     }
   };
-  auto softmax = [&](f32x16& s0, f32x16& s1, int kt, V8* pb, float& alpha, bool& rescale) {
+  auto pv = [&](const unsigned char* vs, const V8 (&pb)[2][2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int db = 0; db < kDB; ++db) {
+        const unsigned char* a = vs + v_rd[db] + t * 32 * L::kRowBytes;
+        const s16x4 lo = lds_read_tr16(a);
+        const s16x4 hi = lds_read_tr16(a + 16 * L::kRowBytes);
+        const u32x4 w = {__builtin_bit_cast(u32x2, lo).x, __builtin_bit_cast(u32x2, lo).y,
+                         __builtin_bit_cast(u32x2, hi).x, __builtin_bit_cast(u32x2, hi).y};
+        oacc[db][0] = E::mma16(as_vec8<V8>(w), pb[0][t], oacc[db][0]);
+        oacc[db][1] = E::mma16(as_vec8<V8>(w), pb[1][t], oacc[db][1]);
+      }
+    }
+  };
+  // P = exp2(s - m) of one query block against a fixed max; returns the lane's sum
+  auto weigh = [&](const f32x4 (&s)[4][2], int qq, float m, V8 (&pb)[2][2]) -> float {
+    float rs = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][qq][j], p.scale_log2, -m));
+        rs += e;
+        pb[qq][kb >> 1][(kb & 1) * 4 + j] = static_cast<typename E::elem>(e);
+      }
+    return rs;
+  };
+  // The general softmax of a tile: masks keys outside the sequence, moves the running maxima
+  // that a tile exceeds by more than `slack`.
+  auto softmax = [&](f32x4 (&s)[4][2], int kt, V8 (&pb)[2][2], float (&alpha)[2], bool& rescale,
+                     float slack = kRescaleSlack) {
     if constexpr (kRagged) {
       const int key0 = p.origin + kt * kBN;
       if (key0 < 0 || key0 + kBN > p.kv_len) {
-        // element i of s0 is key key0 + 8*half + c, c = 16*(i>>3) + (i&7) (s1: c + 32);
-        // comparing the constant c against per-tile bounds keeps no per-element value live
-        const int lo = -key0 - 8 * half;           // key >= 0       <=> c >= lo
-        const int hi = p.kv_len - key0 - 8 * half; // key < kv_len   <=> c < hi
+        // comparing the constant 16kb + j against per-tile bounds keeps no per-element value live
+        const int lo = -key0 - 4 * g;           // key >= 0       <=> 16kb + j >= lo
+        const int hi = p.kv_len - key0 - 4 * g; // key < kv_len   <=> 16kb + j < hi
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int c = (i >> 3) * 16 + (i & 7);
-          if (c < lo || c >= hi) s0[i] = -INFINITY;
-          if (c + 32 < lo || c + 32 >= hi) s1[i] = -INFINITY;
-        }
+        for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const bool out = 16 * kb + j < lo || 16 * kb + j >= hi;
+            s[kb][0][j] = out ? -INFINITY : s[kb][0][j];
+            s[kb][1][j] = out ? -INFINITY : s[kb][1][j];
+          }
       }
     }
-    float mx = s0[0];
+    bool any = false;
 #pragma unroll
-    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s0[i]);
+    for (int qq = 0; qq < 2; ++qq) {
+      float mx = s[0][qq][0];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s1[i]);
-    mx = max_over_halves(mx);
-    const float mxs = mx * p.scale_log2;
-    const bool need = mxs > m_run + kRescaleSlack;
-    rescale = __ballot(need) != 0ull;
-    const float m_new = need ? mxs : m_run;
-    // exp2(0) = 1 when the max is kept; fminf drops the NaN of -inf - -inf
-    alpha = __builtin_amdgcn_exp2f(__builtin_fminf(m_run - m_new, 0.f));
-    m_run = m_new;
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-    float rs = 0.f;
+      for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[i], p.scale_log2, -m_use));
-      const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s1[i], p.scale_log2, -m_use));
-      rs += e0 + e1;
-      pb[i >> 3][i & 7] = static_cast<typename E::elem>(e0);
-      pb[2 + (i >> 3)][i & 7] = static_cast<typename E::elem>(e1);
+        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[kb][qq][j]);
+      mx = max_over_groups(mx);
+      const float mxs = mx * p.scale_log2;
+      const bool need = mxs > m_run[qq] + slack;
+      any = any || need;
+      const float m_new = need ? mxs : m_run[qq];
+      // exp2(0) = 1 when the max is kept; fminf drops the NaN of -inf - -inf
+      alpha[qq] = __builtin_amdgcn_exp2f(__builtin_fminf(m_run[qq] - m_new, 0.f));
+      m_run[qq] = m_new;
+      const float rs = weigh(s, qq, m_new == -INFINITY ? 0.f : m_new, pb);
+      l_run[qq] = l_run[qq] * alpha[qq] + rs;
     }
-    l_run = l_run * alpha + rs;
+    rescale = __ballot(any) != 0ull;
+  };
+  // A tile against the maxima as they are. False, with nothing changed but pb, if some lane's
+  // sum is not below the limit (or the max is still -inf, or a score is NaN): the tile then
+  // takes the general softmax.
+  auto softmax_kept = [&](const f32x4 (&s)[4][2], V8 (&pb)[2][2]) -> bool {
+    const float r0 = weigh(s, 0, m_run[0], pb);
+    const float r1 = weigh(s, 1, m_run[1], pb);
+    const bool ok = __ballot(!(r0 + r1 < kMaxWeightSum)) == 0ull;
+    if (ok) {
+      l_run[0] += r0;
+      l_run[1] += r1;
+    }
+    return ok;
+  };
+  auto rescale_o = [&](const float (&alpha)[2]) {
+#pragma unroll
+    for (int db = 0; db < kDB; ++db) {
+      oacc[db][0] *= alpha[0];
+      oacc[db][1] *= alpha[1];
+    }
   };
 
   // ---- prologue: K_0, V_0 -> stage 0, K_1 -> K stage 1; S_0 -> P_0 ----
-  V8 pb[4];
+  V8 pb[2][2];
   bool act_cur = false;
   int e_n1 = 0, e_n2 = 0;
   if (n_iter > 0) {
@@ -349,11 +402,11 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     __syncthreads();
     act_cur = (f0 & wbit) != 0;
     if (act_cur) {
-      f32x16 s0, s1;
-      qk(k_ring, s0, s1);
-      float alpha;
+      f32x4 s[4][2];
+      qk(k_ring, s);
+      float alpha[2];
       bool rescale;
-      softmax(s0, s1, kt0, pb, alpha, rescale);
+      softmax(s, kt0, pb, alpha, rescale);
     }
     __syncthreads();  // K stage 0 is refilled by the first iteration
   }
@@ -361,7 +414,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   // Iteration j: S_{j+1} = K_{j+1} Q^T, O += P_j V_j, P_{j+1} = softmax(S_{j+1}); K_{j+2}
   // and V_{j+1} stream into the stages freed by iteration j-1.
   bool pend = false;
-  float pend_alpha = 1.f;
+  float pend_alpha[2] = {1.f, 1.f};
   for (int j = 0; j < n_iter; ++j) {
     const bool has1 = j + 1 < n_iter;
     const bool has2 = j + 2 < n_iter;
@@ -375,27 +428,40 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     __builtin_amdgcn_sched_barrier(0);
 
     if (pend) {
-#pragma unroll
-      for (int dsub = 0; dsub < kDSub; ++dsub) oacc[dsub] *= pend_alpha;
+      rescale_o(pend_alpha);
       pend = false;
     }
     const bool act_next = has1 && ((f1 & wbit) != 0);
     const unsigned char* vs = v_ring + (j & 1) * L::kTileBytes;
     const unsigned char* ks1 = k_ring + ((j + 1) & 1) * L::kTileBytes;
-    if (act_cur && act_next) {
-      f32x16 s0, s1;
-      qk(ks1, s0, s1);
+    bool edge = false;  // the next tile crosses token 0 or the sequence end
+    if constexpr (kRagged) {
+      const int key0 = p.origin + kt1 * kBN;
+      edge = key0 < 0 || key0 + kBN > p.kv_len;
+    }
+    if (act_cur && act_next && !edge) {
+      f32x4 s[4][2];
+      qk(ks1, s);
+      // left to itself the scheduler spreads the S products over the P.V and softmax part,
+      // which then waits for them: 2-3 % slower and 20 registers more at D = 128
+      __builtin_amdgcn_sched_barrier(0);
       pv(vs, pb);
-      V8 pn[4];
-      softmax(s0, s1, kt1, pn, pend_alpha, pend);
+      V8 pn[2][2];
+      if (__builtin_expect(!softmax_kept(s, pn), 0)) {
+        qk(ks1, s);
+        softmax(s, kt1, pn, pend_alpha, pend, 0.f);
+      }
 #pragma unroll
-      for (int c = 0; c < 4; ++c) pb[c] = pn[c];
+      for (int t = 0; t < 2; ++t) {
+        pb[0][t] = pn[0][t];
+        pb[1][t] = pn[1][t];
+      }
     } else {
       if (act_cur) pv(vs, pb);
       if (act_next) {
-        f32x16 s0, s1;
-        qk(ks1, s0, s1);
-        softmax(s0, s1, kt1, pb, pend_alpha, pend);
+        f32x4 s[4][2];
+        qk(ks1, s);
+        softmax(s, kt1, pb, pend_alpha, pend);
       }
     }
     act_cur = act_next;
@@ -404,47 +470,42 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     e_n1 = e_n2;
     e_n2 = e_n3;
   }
-  if (pend) {
-#pragma unroll
-    for (int dsub = 0; dsub < kDSub; ++dsub) oacc[dsub] *= pend_alpha;
-  }
+  if (pend) rescale_o(pend_alpha);
 
   // ---- epilogue ----
-  const float l_tot = sum_over_halves(l_run);
+  float l_tot[2];
+#pragma unroll
+  for (int qq = 0; qq < 2; ++qq) l_tot[qq] = sum_over_groups(l_run[qq]);
   if constexpr (kSplit) {
-    const int64_t row = static_cast<int64_t>(blockIdx.x) * kBM + wave * 32 + c32;
-    float* po = p.part_o + row * D;
 #pragma unroll
-    for (int dsub = 0; dsub < kDSub; ++dsub)
+    for (int qq = 0; qq < 2; ++qq) {
+      const int64_t row = static_cast<int64_t>(blockIdx.x) * kBM + wave * 32 + 16 * qq + c16;
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<f32x4*>(po + dsub * 32 + 8 * g + 4 * half) =
-            f32x4{oacc[dsub][4 * g], oacc[dsub][4 * g + 1], oacc[dsub][4 * g + 2], oacc[dsub][4 * g + 3]};
-    if (half == 0) {
-      p.part_ml[2 * row] = m_run;
-      p.part_ml[2 * row + 1] = l_tot;
+      for (int db = 0; db < kDB; ++db)
+        *reinterpret_cast<f32x4*>(p.part_o + row * D + db * 16 + 4 * g) = oacc[db][qq];
+      if (g == 0) {
+        p.part_ml[2 * row] = m_run[qq];
+        p.part_ml[2 * row + 1] = l_tot[qq];
+      }
     }
     return;
   }
-  if (q_row >= 0 && q_row < p.q_len) {
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+#pragma unroll
+  for (int qq = 0; qq < 2; ++qq) {
+    const int q_row = q_row0 + 16 * qq;
+    if (q_row < 0 || q_row >= p.q_len) continue;
+    const float inv = l_tot[qq] > 0.f ? 1.f / l_tot[qq] : 0.f;
     uint16_t* orow = p.o + b * p.o_sb + h * p.o_sh + q_row * p.o_ss;
 #pragma unroll
-    for (int dsub = 0; dsub < kDSub; ++dsub) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d = dsub * 32 + 8 * g + 4 * half;
-        u32x2 w;
-        w.x = pack2(E::from_float(oacc[dsub][4 * g + 0] * inv),
-                    E::from_float(oacc[dsub][4 * g + 1] * inv));
-        w.y = pack2(E::from_float(oacc[dsub][4 * g + 2] * inv),
-                    E::from_float(oacc[dsub][4 * g + 3] * inv));
-        *reinterpret_cast<u32x2*>(orow + d) = w;
-      }
+    for (int db = 0; db < kDB; ++db) {
+      u32x2 w;
+      w.x = pack2(E::from_float(oacc[db][qq][0] * inv), E::from_float(oacc[db][qq][1] * inv));
+      w.y = pack2(E::from_float(oacc[db][qq][2] * inv), E::from_float(oacc[db][qq][3] * inv));
+      *reinterpret_cast<u32x2*>(orow + db * 16 + 4 * g) = w;
     }
-    if (p.lse != nullptr && half == 0) {
+    if (p.lse != nullptr && g == 0) {
       const int64_t li = static_cast<int64_t>(bh) * p.q_len + q_row;
-      p.lse[li] = l_tot > 0.f ? (m_run + log2f(l_tot)) * 0.69314718055994531f : -INFINITY;
+      p.lse[li] = l_tot[qq] > 0.f ? (m_run[qq] + log2f(l_tot[qq])) * 0.69314718055994531f : -INFINITY;
     }
   }
 
@@ -456,23 +517,26 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     // (or all four, for 128-blocks) are whole map cells.
     const int vrow_tile = p.origin + qt * kBM - p.map_q_off;  // multiple of 128
     if (vrow_tile + kBM <= 0 || vrow_tile >= p.map_valid) return;  // uniform per workgroup
-    const int vrow = vrow_tile + wave * 32 + c32;
-    const bool row_ok = vrow >= 0 && vrow < p.map_valid;
-    // the LSE exactly as stored above
-    const float lse_row = l_tot > 0.f ? (m_run + log2f(l_tot)) * 0.69314718055994531f : -INFINITY;
-    const float thr = row_ok ? lse_row + p.map_log_thr : -INFINITY;
-    {
+    float thr[2];
+#pragma unroll
+    for (int qq = 0; qq < 2; ++qq) {
+      const int vrow = vrow_tile + wave * 32 + 16 * qq + c16;
+      const bool row_ok = vrow >= 0 && vrow < p.map_valid;
+      // the LSE exactly as stored above
+      const float lse_row = l_tot[qq] > 0.f ? (m_run[qq] + log2f(l_tot[qq])) * 0.69314718055994531f : -INFINITY;
+      thr[qq] = row_ok ? lse_row + p.map_log_thr : -INFINITY;
       // q scaled in fp32 and rounded to the storage type (reference :86-92)
+      const int q_row = q_row0 + 16 * qq;
       const int r = q_row < 0 ? 0 : (q_row < p.q_len ? q_row : p.q_len - 1);
       const u32x4* src = reinterpret_cast<const u32x4*>(qb + r * p.q_ss);
 #pragma unroll
-      for (int c = 0; c < kDChunks; ++c) {
-        const u32x4 raw = src[2 * c + half];
+      for (int c = 0; c < kKC; ++c) {
+        const u32x4 raw = src[4 * c + g];
         uint16_t e[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) e[j] = E::from_float(E::to_float(u16_at(raw, j)) * p.map_scale);
-        qf[c] = as_vec8<V8>(u32x4{pack2(e[0], e[1]), pack2(e[2], e[3]), pack2(e[4], e[5]),
-                                  pack2(e[6], e[7])});
+        qf[qq][c] = as_vec8<V8>(u32x4{pack2(e[0], e[1]), pack2(e[2], e[3]), pack2(e[4], e[5]),
+                                      pack2(e[6], e[7])});
       }
     }
     // K-only pass: all four 16 KB stages of the K and V rings form one K ring, filled
@@ -497,24 +561,18 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
       // stage (j+3)%4 held tile j-1, read in the previous iteration (barrier since)
       if (j + 3 < n_vt) dma_k(p.map_kt0 + j + 3, (j + 3) & 3);
       __builtin_amdgcn_sched_barrier(0);
-      f32x16 s0, s1;
-      qk(k_ring + (j & 3) * L::kTileBytes, s0, s1);
+      f32x4 s[4][2];
+      qk(k_ring + (j & 3) * L::kTileBytes, s);
       int total = 0;
-      if (j * kBN + kBN > p.map_valid) {
-        // keys past the sequence end are not counted
+      const bool last = j * kBN + kBN > p.map_valid;  // keys past the sequence end are not counted
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int kr = j * kBN + (i >> 3) * 16 + 8 * half + (i & 7);
-          total += __builtin_popcountll(__ballot(s0[i] < thr && kr < p.map_valid));
-          total += __builtin_popcountll(__ballot(s1[i] < thr && kr + 32 < p.map_valid));
-        }
-      } else {
+      for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          total += __builtin_popcountll(__ballot(s0[i] < thr));
-          total += __builtin_popcountll(__ballot(s1[i] < thr));
+        for (int i = 0; i < 4; ++i) {
+          const bool in = !last || j * kBN + 16 * kb + 4 * g + i < p.map_valid;
+          total += __builtin_popcountll(__ballot(s[kb][0][i] < thr[0] && in));
+          total += __builtin_popcountll(__ballot(s[kb][1][i] < thr[1] && in));
         }
-      }
       if (lane == 0) cnt[wave * 2 * kMapFlush + (j % (2 * kMapFlush))] = total;
       // tile j+1 must have landed; the DMAs of tiles j+2 and j+3 (and any map stores,
       // which are younger than tile j+1's DMA) may stay outstanding

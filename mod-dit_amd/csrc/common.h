@@ -133,6 +133,16 @@ __device__ __forceinline__ float sum_over_halves(float x) {
   return __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
 }
 
+// Max / sum of x over lanes l, l ^ 16, l ^ 32 and l ^ 48, in all four.
+__device__ __forceinline__ float max_over_groups(float x) {
+  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return max_over_halves(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])));
+}
+__device__ __forceinline__ float sum_over_groups(float x) {
+  const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return sum_over_halves(__uint_as_float(sw[0]) + __uint_as_float(sw[1]));
+}
+
 template <typename V>
 __device__ __forceinline__ V as_vec8(u32x4 x) {
   return __builtin_bit_cast(V, x);

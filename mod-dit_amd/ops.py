@@ -79,6 +79,10 @@ class TileList:
         return (bits * valid).sum(dim=(1, 2))
 
 
+# The library never splits the key range below 16 key tiles: small calls are spared the question.
+_SPLIT_KEYS = 15 * 64
+
+
 def _workspace(nbytes: int, device):
     """(buffer, size) for a launch that can use `nbytes` of scratch: its own for each call, on
     the current stream. Where the memory is not to be had, the launch runs without."""
@@ -117,13 +121,17 @@ def _attention(q, k, v, scale, return_lse, tiles: TileList | None, out=None):
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _ptr(lse), B, H, Sq, Skv, D,
             strides3(*q.stride()[:3]), strides3(*k.stride()[:3]), strides3(*v.stride()[:3]),
             strides3(*out.stride()[:3]), float(scale), dt)
+    ws, nbytes = None, 0
+    may_split = Skv > _SPLIT_KEYS
     if tiles is None:
-        ws, nbytes = _workspace(lib.moddit_flash_fwd_workspace_bytes(B, H, Sq, Skv, D), q.device)
+        if may_split:
+            ws, nbytes = _workspace(lib.moddit_flash_fwd_workspace_bytes(B, H, Sq, Skv, D), q.device)
         check(lib.moddit_flash_fwd_ws(*args, _ptr(ws), nbytes, _stream(q)), "moddit_flash_fwd")
     else:
-        ws, nbytes = _workspace(
-            lib.moddit_block_sparse_fwd_workspace_bytes(B, H, Sq, D, tiles.cap, int(tiles.origin)),
-            q.device)
+        if may_split:
+            ws, nbytes = _workspace(
+                lib.moddit_block_sparse_fwd_workspace_bytes(B, H, Sq, D, tiles.cap, int(tiles.origin)),
+                q.device)
         check(lib.moddit_block_sparse_fwd_ws(*args, tiles.counts.data_ptr(),
                                              tiles.entries.data_ptr(), tiles.n_qtiles, tiles.cap,
                                              int(tiles.origin), _ptr(ws), nbytes, _stream(q)),
