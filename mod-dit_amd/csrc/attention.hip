@@ -176,7 +176,10 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     else
       it0 = first;
   }
-  const int wbit = 1 << (wave >> 1);
+  // A wave whose 32 rows are all padding takes part in the staging only: 2 of the 52 waves of a
+  // head of 1,577 tokens, two of the four of a 41-row tail.
+  const int first_row = p.origin + qt * kBM + __builtin_amdgcn_readfirstlane(wave) * 32;
+  const int wbit = first_row < p.q_len && first_row + 31 >= 0 ? 1 << (wave >> 1) : 0;
 
   // ---- Q fragments (B operand of S^T = K Q^T): lane holds query 16qq + c16, dims 32c + 8g.. ----
   // Grid rows outside [0, q_len) are padding: they load a clamped row and store nothing.
@@ -441,11 +444,15 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     }
     if (act_cur && act_next && !edge) {
       f32x4 s[4][2];
+      // D = 128: left to itself the scheduler spreads the S products over the P.V and softmax
+      // part, which then waits for them: 2-3 % slower and 20 registers more. D = 64: half the
+      // products and as much softmax, which starts sooner after P.V (1 % on short sweeps).
+      if constexpr (D == 64) pv(vs, pb);
       qk(ks1, s);
-      // left to itself the scheduler spreads the S products over the P.V and softmax part,
-      // which then waits for them: 2-3 % slower and 20 registers more at D = 128
-      __builtin_amdgcn_sched_barrier(0);
-      pv(vs, pb);
+      if constexpr (D == 128) {
+        __builtin_amdgcn_sched_barrier(0);
+        pv(vs, pb);
+      }
       V8 pn[2][2];
       if (__builtin_expect(!softmax_kept(s, pn), 0)) {
         qk(ks1, s);
