@@ -8,10 +8,11 @@
 //   O^T (D x 32 queries)      += V8^T . P8^T   mfma_f32_32x32x64 fp8  (D/32 per tile)
 // A tile is D bytes per key for K and for V, so a 3-stage ring takes 48 KB of LDS at
 // D=128: K tiles are fetched three tiles ahead, V tiles two, each into the stage its
-// predecessor three tiles back left free at the previous barrier. 48 KB and 166 VGPRs
-// let three workgroups share a CU (three waves per SIMD) in the aligned and in the dense
-// ragged kernels. The block-sparse ragged kernels convert the scores once and mask boundary
-// tiles in place: 137 VGPRs at D=64 (three waves), 197 at D=128 (two; three would spill).
+// predecessor three tiles back left free at the previous barrier. 48 KB and 164-168 VGPRs
+// let three workgroups share a CU (three waves per SIMD) at D=128 in the aligned and the
+// dense ragged kernels, 24 KB and 126-127 VGPRs four at D=64. The block-sparse ragged kernels
+// convert the scores once and mask boundary tiles in place: 137 VGPRs at D=64 (three waves),
+// 197 at D=128 (two; three would spill).
 //
 // Operand layouts. MFMA products are sums over k, so any assignment of (lane half, byte)
 // to k works as long as both operands use the same one; the layouts below are chosen so
@@ -30,6 +31,7 @@
 #include "common.h"
 #include "lds_dma.h"
 
+#include <climits>
 #include <type_traits>
 
 namespace moddit {
@@ -96,8 +98,19 @@ template <int D>
 __device__ __forceinline__ int swz_k8(int r) { return (r / (256 / D)) % (D / 16); }
 __device__ __forceinline__ int swz_v8(int r) { return (r >> 2) & 3; }
 
+// What a tile's softmax masks: nothing, keys from seq_len on, or keys outside [0, seq_len)
+// where the tile crosses either.
+enum class Edge { kNone, kEnd, kBoth };
+
+// Waves per SIMD that the registers are held to (the aligned kernels at D = 64 fit four
+// without being held to it; the dense ragged one needs 129 registers left to itself).
+constexpr int q8_waves(int head_dim, bool sparse, bool ragged) {
+  if (ragged && sparse) return head_dim == 128 ? 2 : 3;
+  return ragged && head_dim == 64 ? 4 : 3;
+}
+
 template <int D, typename E, bool kSparse, bool kRagged>
-__global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3) __attribute__((amdgpu_waves_per_eu((kRagged && kSparse && D == 128) ? 2 : 3, (kRagged && kSparse && D == 128) ? 2 : 3))) void attention_q8_kernel(Q8Params p) {
+__global__ __launch_bounds__(kThreads, q8_waves(D, kSparse, kRagged)) __attribute__((amdgpu_waves_per_eu(q8_waves(D, kSparse, kRagged), q8_waves(D, kSparse, kRagged)))) void attention_q8_kernel(Q8Params p) {
   using L = Q8Lds<D>;
   constexpr int kKSteps = D / 32;                // int8 MFMA k-steps over d
   constexpr int kDSub = D / 32;                  // 32-row blocks of O^T
@@ -253,19 +266,30 @@ __global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3)
   };
   // scores of key tile kt: s = int32 * q_scale * k_scale[kt], in log2 units (the softmax
   // scale is folded into q_sc)
-  auto softmax_of = [&](auto edge, const i32x16& s0, const i32x16& s1, int kt, i32x8& pb,
-                        float& alpha, bool& rescale) {
-    constexpr bool kEdge = decltype(edge)::value;  // the tile may cross 0 or seq_len
+  auto softmax = [&](auto edge, i32x16& s0, i32x16& s1, int kt, i32x8& pb, float& alpha,
+                     bool& rescale) {
+    constexpr Edge kEdge = decltype(edge)::value;
     const int key0 = p.origin + kt * kBN;
     float f0[16], f1[16];
     float mx;
     bool general = false;
     // tiles wholly inside the sequence share one K scale on any grid (the quantiser's
     // blocks lie on the attention grid), so only tiles that cross 0 or seq_len need masking
-    if constexpr (kEdge) general = key0 < 0 || key0 + kBN > p.seq_len;
+    if constexpr (kEdge == Edge::kBoth) general = key0 < 0 || key0 + kBN > p.seq_len;
     const float sc = kscale[kt] * q_sc;  // one K scale per tile on any grid, q_sc > 0
-    if constexpr (!kEdge) {
-      // every tile inside the sequence: max over the raw integer scores
+    if constexpr (kEdge != Edge::kBoth) {
+      // element i of s0 is key key0 + 32*half + i (s1: + 16); those from seq_len on take no
+      // part in the max here, and in P and the row sum below. The tile holds at least one key
+      // of the sequence, so the row's max is a real one.
+      const int hi = p.seq_len - key0 - 32 * half;
+      if constexpr (kEdge == Edge::kEnd) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          if (i >= hi) s0[i] = INT_MIN;
+          if (i + 16 >= hi) s1[i] = INT_MIN;
+        }
+      }
+      // max over the raw integer scores
       int mi = s0[0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) mi = max(mi, s0[i]);
@@ -293,9 +317,13 @@ __global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3)
       for (int i = 0; i < 16; ++i) {
         f0[i] = __builtin_fmaf(f0[i], sc, -m_sh);
         f1[i] = __builtin_fmaf(f1[i], sc, -m_sh);
+        if constexpr (kEdge == Edge::kEnd) {
+          if (i >= hi) f0[i] = -INFINITY;
+          if (i + 16 >= hi) f1[i] = -INFINITY;
+        }
       }
     } else {
-      // ragged grids: the scores are converted once and, on tiles that cross 0 or
+      // lists on ragged grids: the scores are converted once and, on tiles that cross 0 or
       // seq_len, masked in place, so both paths share the same registers
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
@@ -366,19 +394,16 @@ __global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3)
     }
     l_run = l_run * alpha + rs;
   };
-  // Masking boundary tiles inside the loop costs registers (199 VGPRs at D = 128: two waves
-  // per SIMD instead of three). A dense sweep has one boundary tile, its last, and does
-  // without: its keys past the end have K = 0 and V = 0, so a score of 0 and no part in O.
-  // They can move the running max only where every key's score is below -kRescaleSlack,
-  // which K minus its mean over the sequence does not allow (a row's scores add up to 0 but
-  // for their rounding), and their share of the row sum is taken out after the loop. Lists
-  // may name a boundary tile anywhere and few other keys, so they are masked. Dense, 17,776
-  // keys x 48 heads, D = 64: 3.75 -> 3.45 ms; 28,776 x 24, D = 128: 7.19 -> 6.5 ms.
-  constexpr bool kMaskInLoop = kRagged && kSparse;
-  auto softmax = [&](const i32x16& s0, const i32x16& s1, int kt, i32x8& pb, float& alpha,
-                     bool& rescale) {
-    softmax_of(std::bool_constant<kMaskInLoop>{}, s0, s1, kt, pb, alpha, rescale);
-  };
+  // Masking boundary tiles inside the loop costs registers (197 VGPRs at D = 128: two waves
+  // per SIMD instead of three). A dense sweep has one boundary tile, its last, so its loop
+  // masks nothing and its last two iterations are a copy of the loop's body that does
+  // (17,776 keys x 48 heads, D = 64: 3.31 ms against 3.75 masked in the loop; 28,776 x 24, D =
+  // 128: 6.3 against 7.19). Letting the padding take part (K = 0: a score of 0) and taking it
+  // out of the row sum afterwards is not an option: int8 rounding can leave a row whose real
+  // scores are all far below 0. Lists may name a boundary tile anywhere: masked inside.
+  constexpr bool kMaskLast = kRagged && !kSparse;
+  using InLoop = std::integral_constant<Edge, kRagged && kSparse ? Edge::kBoth : Edge::kNone>;
+  using AtEnds = std::integral_constant<Edge, kMaskLast ? Edge::kEnd : InLoop::value>;
 
   // ---- prologue: K_0..K_2 -> K stages 0..2, V_0, V_1 -> V stages 0, 1; S_0 -> P_0 ----
   i32x8 pb = i32x8{};
@@ -412,7 +437,7 @@ __global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3)
       qk(k_ring, s0, s1);
       float alpha;
       bool rescale;
-      softmax_of(std::bool_constant<kRagged>{}, s0, s1, kt0, pb, alpha, rescale);
+      softmax(AtEnds{}, s0, s1, kt0, pb, alpha, rescale);
     }
     __syncthreads();  // K stage 0 is refilled by the first iteration
   }
@@ -423,7 +448,7 @@ __global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3)
   bool pend = false;
   float pend_alpha = 1.f;
   int st0 = 0, st1 = 1, st2 = 2;  // ring stages of tiles j, j+1, j+2; tile j+3 reuses st0
-  for (int j = 0; j < n_iter; ++j) {
+  auto iterate = [&](auto edge, int j) {
     const bool has1 = j + 1 < n_iter;
     const bool has2 = j + 2 < n_iter;
     const bool has3 = j + 3 < n_iter;
@@ -449,13 +474,13 @@ __global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3)
       i32x16 s0, s1;
       qk(ks1, s0, s1);
       pv(vs, pb);
-      softmax(s0, s1, kt1, pb, pend_alpha, pend);  // P_{j+1} overwrites P_j after its MFMAs
+      softmax(edge, s0, s1, kt1, pb, pend_alpha, pend);  // P_{j+1} overwrites P_j after its MFMAs
     } else {
       if (act_cur) pv(vs, pb);
       if (act_next) {
         i32x16 s0, s1;
         qk(ks1, s0, s1);
-        softmax(s0, s1, kt1, pb, pend_alpha, pend);
+        softmax(edge, s0, s1, kt1, pb, pend_alpha, pend);
       }
     }
     act_cur = act_next;
@@ -475,19 +500,16 @@ __global__ __launch_bounds__(kThreads, (kRagged && kSparse && D == 128) ? 2 : 3)
     st0 = st1;
     st1 = st2;
     st2 = freed;
+  };
+  int j = 0;
+  for (; j < (kMaskLast ? n_iter - 2 : n_iter); ++j) iterate(InLoop{}, j);
+  if constexpr (kMaskLast) {
+#pragma unroll 1
+    for (; j < n_iter; ++j) iterate(AtEnds{}, j);
   }
   if (pend) {
 #pragma unroll
     for (int ds = 0; ds < kDSub; ++ds) oacc[ds] *= pend_alpha;
-  }
-
-  if constexpr (kRagged && !kSparse) {
-    // this lane's keys of the last tile past the sequence end added exp2(0 - (m - kPShift)) each
-    if (n_iter > 1) {
-      const int in = p.seq_len - (n_iter - 1) * kBN - 32 * half;
-      const int outside = in >= 32 ? 0 : (in <= 0 ? 32 : 32 - in);
-      l_run -= static_cast<float>(outside) * __builtin_amdgcn_exp2f(kPShift - m_run);
-    }
   }
 
   // ---- epilogue: O = O^T * v_scale[d] / l ----
