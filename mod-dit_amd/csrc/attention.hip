@@ -13,12 +13,13 @@
 // What bounds it is the board's power limit: the clock falls until the power fits, so time
 // follows the energy of the work, not its schedule. The 16x16x32 shape does the same
 // products for less (2.19 against 1.86 PFLOP/s for 32x32x16 on random operands at the
-// limit). Its price, two queries per lane and with them twice the row reductions, is not
-// paid on most tiles: the softmax takes the running max as it is and checks the lane's sum
-// of weights afterwards (softmax_kept). Against the 32x32x16 kernel with a max per tile, on
-// structured inputs: dense 24 heads x 115,200, D = 128 145.9 -> 137.2 ms (1,190 TFLOP/s; a
-// hipBLASLt GEMM of 8,192^3 runs at 1,180 there), block-sparse 40 x 69,120 20.0 -> 19.0 ms,
-// 48 x 17,776, D = 64 1.45 -> 1.41 ms.
+// limit). Its price, two queries per lane and with them twice the row reductions, is kept
+// off most tiles: a lane compares its own scores with the running max, and the row max is
+// exchanged and moved only where one of them lies far above it (settle). Against the 32x32x16
+// kernel with a max per tile, on structured inputs: dense 24 heads x 115,200, D = 128 150.5 ->
+// 144.3 ms; block-sparse 40 x 69,120 20.5 -> 19.7 ms; 48 x 17,776, D = 64 1.51 -> 1.40 ms.
+// Weighing a tile against the max as it is, and computing it again where that overflows, takes
+// the lanes' max off too (143.2, 19.8 and 1.45 ms) but costs peaked rows up to 40 %.
 //
 // K and V tiles go straight from HBM into LDS (buffer_load ... lds, no register
 // staging), both row-major with an XOR swizzle on 16-byte chunks that keeps the operand
@@ -37,6 +38,8 @@
 // fp32 softmax instead of SageAttention's quantisation.
 #include "common.h"
 #include "lds_dma.h"
+
+#include <cfloat>
 
 namespace moddit {
 namespace {
@@ -101,17 +104,11 @@ __device__ __forceinline__ int swz_k(int r) { return (r / (128 / D)) % (D / 8); 
 template <int D>
 __device__ __forceinline__ int swz_v(int key) { return 2 * ((key / (128 / D)) % (D / 16)); }
 
-// The running row max is not looked at on most tiles: a tile's weights are taken against the
-// max as it is, and only if a lane's sum of them reaches kMaxWeightSum does the tile go
-// through the general softmax, which then moves every row's max to the tile's where that is
-// larger. On other tiles that take the general softmax (the first, boundaries, exact rows'
-// gaps) it moves by more than kRescaleSlack log2 units only. Softmax is shift-invariant, so
-// results do not depend on either, but for the rounding of P: a row's largest weight is
-// exact (1) where the max is its own. The limit 256 = 2^kRescaleSlack keeps the error
-// against fp64 at that of a max per tile (2.16e-3 and 2.17e-3 of the result on the
-// Wan-like layer); 1,024 and 2^20 are up to 1 and 2 % faster there, at 2.22e-3 and 2.31e-3.
+// The running maxima move only on tiles where some lane of the wave holds a score more than
+// kRescaleSlack log2 units above its row's; there every row's max moves to the tile's if that
+// is larger. Softmax is shift-invariant, so results do not depend on it but for the rounding of
+// P, whose weights reach 2^kRescaleSlack at most.
 constexpr float kRescaleSlack = 8.0f;
-constexpr float kMaxWeightSum = 256.0f;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -266,7 +263,7 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
   f32x4 oacc[kDB][2];
 #pragma unroll
   for (int db = 0; db < kDB; ++db) oacc[db][0] = oacc[db][1] = f32x4{};
-  float m_run[2] = {-INFINITY, -INFINITY};
+  float m_run[2] = {-FLT_MAX, -FLT_MAX};  // never -inf: no difference of maxima is NaN
   float l_run[2] = {0.f, 0.f};  // this lane's keys only
 
   auto decode = [&](int e_raw, int& kt, int& flags) {
@@ -294,11 +291,13 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
       }
     }
   };
-  auto pv = [&](const unsigned char* vs, const V8 (&pb)[2][2]) {
+  // O += P V: of its 2 kDB steps in the order (t, db), [i0, i1)
+  auto pv = [&](const unsigned char* vs, const V8 (&pb)[2][2], int i0 = 0, int i1 = D / 8) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int db = 0; db < kDB; ++db) {
+        if (t * kDB + db < i0 || t * kDB + db >= i1) continue;
         const unsigned char* a = vs + v_rd[db] + t * 32 * L::kRowBytes;
         const s16x4 lo = lds_read_tr16(a);
         const s16x4 hi = lds_read_tr16(a + 16 * L::kRowBytes);
@@ -309,72 +308,66 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
       }
     }
   };
-  // P = exp2(s - m) of one query block against a fixed max; returns the lane's sum
-  auto weigh = [&](const f32x4 (&s)[4][2], int qq, float m, V8 (&pb)[2][2]) -> float {
-    float rs = 0.f;
+  // Moves the running maxima, and sets alpha and rescale, only where a lane of the wave holds a
+  // score more than kRescaleSlack above its row's max.
+  auto settle = [&](const f32x4 (&s)[4][2], float (&alpha)[2], bool& rescale) {
+    float mx[2];
+#pragma unroll
+    for (int qq = 0; qq < 2; ++qq) {
+      mx[qq] = s[0][qq][0];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mx[qq] = fmaxf(mx[qq], s[kb][qq][j]);
+    }
+    const float over = fmaxf(__builtin_fmaf(mx[0], p.scale_log2, -m_run[0]),
+                             __builtin_fmaf(mx[1], p.scale_log2, -m_run[1]));
+    if (__builtin_expect(__ballot(over > kRescaleSlack) != 0ull, 0)) {
+#pragma unroll
+      for (int qq = 0; qq < 2; ++qq) {
+        const float m_new = fmaxf(m_run[qq], max_over_groups(mx[qq]) * p.scale_log2);
+        alpha[qq] = __builtin_amdgcn_exp2f(m_run[qq] - m_new);
+        l_run[qq] *= alpha[qq];
+        m_run[qq] = m_new;
+      }
+      rescale = true;
+    }
+  };
+  // P = exp2(s - m) and its share of the row sums
+  auto weigh = [&](const f32x4 (&s)[4][2], V8 (&pb)[2][2]) {
+#pragma unroll
+    for (int qq = 0; qq < 2; ++qq) {
+      float rs = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][qq][j], p.scale_log2, -m_run[qq]));
+          rs += e;
+          pb[qq][kb >> 1][(kb & 1) * 4 + j] = static_cast<typename E::elem>(e);
+        }
+      l_run[qq] += rs;
+    }
+  };
+  // keys outside the sequence: a score of -inf
+  auto mask = [&](f32x4 (&s)[4][2], int kt) {
+    const int key0 = p.origin + kt * kBN;
+    // comparing the constant 16kb + j against per-tile bounds keeps no per-element value live
+    const int lo = -key0 - 4 * g;           // key >= 0       <=> 16kb + j >= lo
+    const int hi = p.kv_len - key0 - 4 * g; // key < kv_len   <=> 16kb + j < hi
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][qq][j], p.scale_log2, -m));
-        rs += e;
-        pb[qq][kb >> 1][(kb & 1) * 4 + j] = static_cast<typename E::elem>(e);
+        const bool out = 16 * kb + j < lo || 16 * kb + j >= hi;
+        s[kb][0][j] = out ? -INFINITY : s[kb][0][j];
+        s[kb][1][j] = out ? -INFINITY : s[kb][1][j];
       }
-    return rs;
   };
-  // The general softmax of a tile: masks keys outside the sequence, moves the running maxima
-  // that a tile exceeds by more than `slack`.
-  auto softmax = [&](f32x4 (&s)[4][2], int kt, V8 (&pb)[2][2], float (&alpha)[2], bool& rescale,
-                     float slack = kRescaleSlack) {
-    if constexpr (kRagged) {
-      const int key0 = p.origin + kt * kBN;
-      if (key0 < 0 || key0 + kBN > p.kv_len) {
-        // comparing the constant 16kb + j against per-tile bounds keeps no per-element value live
-        const int lo = -key0 - 4 * g;           // key >= 0       <=> 16kb + j >= lo
-        const int hi = p.kv_len - key0 - 4 * g; // key < kv_len   <=> 16kb + j < hi
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const bool out = 16 * kb + j < lo || 16 * kb + j >= hi;
-            s[kb][0][j] = out ? -INFINITY : s[kb][0][j];
-            s[kb][1][j] = out ? -INFINITY : s[kb][1][j];
-          }
-      }
-    }
-    bool any = false;
-#pragma unroll
-    for (int qq = 0; qq < 2; ++qq) {
-      float mx = s[0][qq][0];
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[kb][qq][j]);
-      mx = max_over_groups(mx);
-      const float mxs = mx * p.scale_log2;
-      const bool need = mxs > m_run[qq] + slack;
-      any = any || need;
-      const float m_new = need ? mxs : m_run[qq];
-      // exp2(0) = 1 when the max is kept; fminf drops the NaN of -inf - -inf
-      alpha[qq] = __builtin_amdgcn_exp2f(__builtin_fminf(m_run[qq] - m_new, 0.f));
-      m_run[qq] = m_new;
-      const float rs = weigh(s, qq, m_new == -INFINITY ? 0.f : m_new, pb);
-      l_run[qq] = l_run[qq] * alpha[qq] + rs;
-    }
-    rescale = __ballot(any) != 0ull;
-  };
-  // A tile against the maxima as they are. False, with nothing changed but pb, if some lane's
-  // sum is not below the limit (or the max is still -inf, or a score is NaN): the tile then
-  // takes the general softmax.
-  auto softmax_kept = [&](const f32x4 (&s)[4][2], V8 (&pb)[2][2]) -> bool {
-    const float r0 = weigh(s, 0, m_run[0], pb);
-    const float r1 = weigh(s, 1, m_run[1], pb);
-    const bool ok = __ballot(!(r0 + r1 < kMaxWeightSum)) == 0ull;
-    if (ok) {
-      l_run[0] += r0;
-      l_run[1] += r1;
-    }
-    return ok;
+  auto crosses_edge = [&](int kt) -> bool {
+    if constexpr (!kRagged) return false;
+    const int key0 = p.origin + kt * kBN;
+    return key0 < 0 || key0 + kBN > p.kv_len;
   };
   auto rescale_o = [&](const float (&alpha)[2]) {
 #pragma unroll
@@ -407,9 +400,11 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     if (act_cur) {
       f32x4 s[4][2];
       qk(k_ring, s);
+      if (crosses_edge(kt0)) mask(s, kt0);
       float alpha[2];
       bool rescale;
-      softmax(s, kt0, pb, alpha, rescale);
+      settle(s, alpha, rescale);
+      weigh(s, pb);
     }
     __syncthreads();  // K stage 0 is refilled by the first iteration
   }
@@ -437,27 +432,23 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
     const bool act_next = has1 && ((f1 & wbit) != 0);
     const unsigned char* vs = v_ring + (j & 1) * L::kTileBytes;
     const unsigned char* ks1 = k_ring + ((j + 1) & 1) * L::kTileBytes;
-    bool edge = false;  // the next tile crosses token 0 or the sequence end
-    if constexpr (kRagged) {
-      const int key0 = p.origin + kt1 * kBN;
-      edge = key0 < 0 || key0 + kBN > p.kv_len;
-    }
-    if (act_cur && act_next && !edge) {
+    if (act_cur && act_next) {
       f32x4 s[4][2];
-      // D = 128: left to itself the scheduler spreads the S products over the P.V and softmax
-      // part, which then waits for them: 2-3 % slower and 20 registers more. D = 64: half the
-      // products and as much softmax, which starts sooner after P.V (1 % on short sweeps).
+      // The P.V steps lie where something else waits. D = 128: some under the max of the new
+      // scores, the others under their weights (10 and 6 of 16; all before: 1-2 % slower where
+      // power does not bound, all after: 2-6 % on large calls); left to itself the scheduler
+      // spreads the S products over them, and the softmax waits. D = 64: half the products and
+      // as much softmax, which starts sooner after P.V; four waves cover the rest.
+      constexpr int kUnderMax = 10;
       if constexpr (D == 64) pv(vs, pb);
       qk(ks1, s);
-      if constexpr (D == 128) {
-        __builtin_amdgcn_sched_barrier(0);
-        pv(vs, pb);
-      }
+      if (crosses_edge(kt1)) mask(s, kt1);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (D == 128) pv(vs, pb, 0, kUnderMax);
+      settle(s, pend_alpha, pend);
+      if constexpr (D == 128) pv(vs, pb, kUnderMax);
       V8 pn[2][2];
-      if (__builtin_expect(!softmax_kept(s, pn), 0)) {
-        qk(ks1, s);
-        softmax(s, kt1, pn, pend_alpha, pend, 0.f);
-      }
+      weigh(s, pn);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         pb[0][t] = pn[0][t];
@@ -468,7 +459,9 @@ __global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 
       if (act_next) {
         f32x4 s[4][2];
         qk(ks1, s);
-        softmax(s, kt1, pb, pend_alpha, pend);
+        if (crosses_edge(kt1)) mask(s, kt1);
+        settle(s, pend_alpha, pend);
+        weigh(s, pb);
       }
     }
     act_cur = act_next;
@@ -646,14 +639,13 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(AttnParams p) {
     const int q_row = p.origin + qt * kBM + r;
     if (q_row < 0 || q_row >= p.q_len) continue;
     const int64_t row0 = static_cast<int64_t>(tile) * p.n_split * kBM + r;
-    float m = -INFINITY;
+    float m = -FLT_MAX;  // the kernels' own start value
     for (int i = 0; i < p.n_split; ++i) m = fmaxf(m, p.part_ml[2 * (row0 + i * kBM)]);
-    const float m_use = m == -INFINITY ? 0.f : m;
     float l = 0.f;
     f32x4 o = f32x4{};
     for (int i = 0; i < p.n_split; ++i) {
       const int64_t row = row0 + i * kBM;
-      const float w = __builtin_amdgcn_exp2f(p.part_ml[2 * row] - m_use);
+      const float w = __builtin_amdgcn_exp2f(p.part_ml[2 * row] - m);
       l += p.part_ml[2 * row + 1] * w;
       o += *reinterpret_cast<const f32x4*>(p.part_o + row * D + d) * w;
     }

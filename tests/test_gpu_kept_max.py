@@ -1,6 +1,6 @@
 """Attention tiles whose weights are taken against an older running max (GPU): scores that
-climb, fall and jump along the keys, so that tiles land on both sides of the limit on the
-lane's weight sum, and non-finite scores, against fp64 attention."""
+climb, fall and jump along the keys, so that tiles land on both sides of the rescale limit,
+and non-finite scores, against fp64 attention."""
 import pytest
 import torch
 
