@@ -110,6 +110,13 @@ __device__ __forceinline__ int swz_v(int key) { return 2 * ((key / (128 / D)) % 
 // P, whose weights reach 2^kRescaleSlack at most.
 constexpr float kRescaleSlack = 8.0f;
 
+// Waves per SIMD that the registers are held to. D = 128 takes 211-227 (two waves). D = 64 fits
+// four in 124-128 (left alone, up to 134; the aligned dense kernel keeps seven invariants of
+// its last tile in scratch), the fused map three. Where a launch has four workgroups per CU,
+// three waves leave a quarter of them to a second round: 8 heads x 16,384, exact rows, a
+// tenth of the tiles: 132 against 104 us.
+constexpr int attn_waves(int head_dim, bool map) { return head_dim == 128 ? 2 : (map ? 3 : 4); }
+
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 // ds_read_b64_tr_b16: within each 16-lane group, lane i receives element i%4 of the
@@ -126,7 +133,7 @@ constexpr int kMapCountBytes = 4 * 2 * kMapFlush * 4;  // int per (wave, ring sl
 // kSplit: one workgroup takes the piece `blockIdx % n_split` of a query tile's key tiles (or
 // list entries) and leaves its unnormalised fp32 O, max and sum for combine_kernel.
 template <int D, typename E, bool kSparse, bool kRagged, bool kMap = false, bool kSplit = false>
-__global__ __launch_bounds__(kThreads, 2) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_fwd_kernel(AttnParams p) {
+__global__ __launch_bounds__(kThreads, attn_waves(D, kMap)) __attribute__((amdgpu_waves_per_eu(attn_waves(D, kMap), attn_waves(D, kMap)))) void attention_fwd_kernel(AttnParams p) {
   using L = AttnLds<D>;
   using V8 = typename E::vec8;
   constexpr int kKC = D / 32;  // MFMA k-steps over d for S^T

@@ -1,5 +1,5 @@
 """Times of bf16/fp16 attention calls relative to each other, in one process (GPU): what
-the scores' spread may cost."""
+neither the scores' spread nor one more workgroup per CU may cost."""
 import pytest
 import torch
 
@@ -39,3 +39,17 @@ def test_peaked_rows_cost_no_second_sweep(H, S, D):
     print(f"H={H} S={S} D={D}: {t0:.1f} us flat, {t1:.1f} us peaked", flush=True)
     assert t1 <= 1.25 * t0, (t0, t1)
 
+
+def test_four_workgroups_share_a_cu_at_d64():
+    """1,024 query tiles (four per CU) against 768 (three): one round each (measured
+    1.11; 1.31 where only three fitted)."""
+    def one(H, S=16384):
+        q, k, v = _qkv(H, S, 64)
+        g = torch.Generator(device="cuda").manual_seed(1)
+        mask = torch.rand((1, S // 64, S // 64), generator=g, device="cuda").expand(H, -1, -1) < 0.1
+        tiles = ops.mask_to_tiles(mask, 64, union_rows=False)
+        return _us(lambda: ops.block_sparse_fwd(q, k, v, tiles))
+
+    t6, t8 = one(6), one(8)
+    print(f"6 heads {t6:.1f} us, 8 heads {t8:.1f} us", flush=True)
+    assert t8 <= 1.2 * t6, (t6, t8)
