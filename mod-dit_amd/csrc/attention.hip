@@ -718,14 +718,16 @@ int launch_attention(const AttnParams& p, int batch, hipStream_t stream) {
 // tail, a short clip, few heads): its time is a whole key sweep however few they are. The
 // sweep is then split over `n_split` workgroups per tile, at the price of writing and
 // re-reading fp32 partial outputs and one more launch. The choice compares estimates of
-// both, from the time a key tile takes with k workgroups on a CU (measured: D = 128
-// 1.48 / 2.18 / 3.49 / 4.20 us, D = 64 1.11 / 1.45 / 2.06 / 2.53 us for k = 1..4, and
-// 1.04 k and 0.61 k beyond). List lengths are known on the device only: a block-sparse
-// list is taken to hold a quarter of its capacity. Against the best of 1..32 pieces the
-// choice is within 5 % over 21 shapes; e.g. 256 text rows x 24 heads over 29,019 keys, D =
-// 128 (48 tiles): 650 us unsplit, 136 us in 10 pieces; over 115,419 keys 2,551 and 492 us;
-// 4,096 tokens x 2 heads, D = 64 (64 tiles): 70 and 30 us. From about one tile per CU on
-// the split no longer pays (432 tiles of 36 key tiles: 39 us unsplit, 59 us in two).
+// both, from the time a key tile takes with k workgroups on a CU (cu_tile_us: fitted to 166
+// measured shapes of 1 to 512 query tiles by 16 to 512 key tiles, 1 to 32 pieces each). List
+// lengths are known on the device only: a block-sparse list is taken to hold a quarter of its
+// capacity. On those shapes the choice is never slower than no split, on average 3.5 % from
+// the best of 1..32 pieces and at worst 25 % (sweeps of 16 key tiles, which are kept at two
+// pieces): 256 text rows x 24 heads over 29,019 keys, D = 128 (48 tiles): 614 us unsplit,
+// 129 in 10 pieces; over 115,419 keys 2,414 and 455 us; 4,096 tokens x 2 heads, D = 64 (64
+// tiles): 66 and 29 us. Two tiles per CU no longer gain (432 tiles of 36 key tiles: 46 us
+// unsplit, 58 us in two). A list that holds less than a twentieth of its capacity loses the
+// second launch, 4 us (32 tiles of one entry, D = 64: 13.4 -> 17.5 us a call).
 constexpr int kMaxSplit = 64;
 // Key tiles per piece at the least: below 16 key tiles the second launch costs a dense call
 // what the split saves. A list's estimate is rough: real lists
@@ -734,8 +736,9 @@ constexpr int kMinPieceDense = 8;
 constexpr int kMinPieceSparse = 4;
 
 double cu_tile_us(int head_dim, int64_t k) {
-  if (head_dim == 128) return 1.05 * k + (k % 2 ? 0.38 : 0.08);
-  return 0.61 * k + (k == 1 ? 0.5 : 0.2);
+  constexpr double k128[4] = {1.33, 1.81, 3.14, 4.05}, k64[4] = {0.97, 1.17, 1.72, 2.19};
+  if (head_dim == 128) return k <= 4 ? k128[k - 1] : k128[3] + 1.01 * (k - 4);
+  return k <= 4 ? k64[k - 1] : k64[3] + 0.46 * (k - 4);
 }
 
 int split_for(int64_t tiles, int64_t key_tiles, int min_piece, int head_dim) {
@@ -747,7 +750,7 @@ int split_for(int64_t tiles, int64_t key_tiles, int min_piece, int head_dim) {
     const int64_t per_cu = static_cast<int64_t>((tiles * s + kCus - 1) / kCus);
     double us = cu_tile_us(head_dim, per_cu) * (static_cast<double>(key_tiles) / s + kFixedTiles);
     if (s > 1) us += kLaunchUs + tiles * s * (kBM * (head_dim + 2) * 8.0) / kPartialBytesPerUs;
-    if (s == 1 || us < 0.95 * best_us) {
+    if (s == 1 || us < 0.97 * best_us) {
       best = s;
       best_us = us;
     }
