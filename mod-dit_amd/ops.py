@@ -6,6 +6,7 @@ Nothing in this module computes on the host, and nothing falls back to torch mat
 """
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass
 
@@ -79,8 +80,11 @@ class TileList:
         return (bits * valid).sum(dim=(1, 2))
 
 
-# The library never splits the key range below 16 key tiles: small calls are spared the question.
-_SPLIT_KEYS = 15 * 64
+@functools.lru_cache(maxsize=1024)
+def _split_bytes(query: str, *sizes: int) -> int:
+    """The library's answer (0: none) to one of its *_workspace_bytes queries: a function of the
+    sizes alone."""
+    return getattr(_lib.load(), query)(*sizes)
 
 
 def _workspace(nbytes: int, device):
@@ -121,17 +125,14 @@ def _attention(q, k, v, scale, return_lse, tiles: TileList | None, out=None):
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _ptr(lse), B, H, Sq, Skv, D,
             strides3(*q.stride()[:3]), strides3(*k.stride()[:3]), strides3(*v.stride()[:3]),
             strides3(*out.stride()[:3]), float(scale), dt)
-    ws, nbytes = None, 0
-    may_split = Skv > _SPLIT_KEYS
     if tiles is None:
-        if may_split:
-            ws, nbytes = _workspace(lib.moddit_flash_fwd_workspace_bytes(B, H, Sq, Skv, D), q.device)
+        ws, nbytes = _workspace(
+            _split_bytes("moddit_flash_fwd_workspace_bytes", B, H, Sq, Skv, D), q.device)
         check(lib.moddit_flash_fwd_ws(*args, _ptr(ws), nbytes, _stream(q)), "moddit_flash_fwd")
     else:
-        if may_split:
-            ws, nbytes = _workspace(
-                lib.moddit_block_sparse_fwd_workspace_bytes(B, H, Sq, D, tiles.cap, int(tiles.origin)),
-                q.device)
+        ws, nbytes = _workspace(
+            _split_bytes("moddit_block_sparse_fwd_workspace_bytes", B, H, Sq, D, tiles.cap,
+                         int(tiles.origin)), q.device)
         check(lib.moddit_block_sparse_fwd_ws(*args, tiles.counts.data_ptr(),
                                              tiles.entries.data_ptr(), tiles.n_qtiles, tiles.cap,
                                              int(tiles.origin), _ptr(ws), nbytes, _stream(q)),

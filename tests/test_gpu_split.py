@@ -109,3 +109,21 @@ def test_split_replays_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         ops.flash_fwd(k, q, v[:, :, :256])
+
+
+@pytest.mark.parametrize("op", ["flash_fwd", "block_sparse_fwd"])
+def test_the_library_decides_what_splits(op, monkeypatch):
+    """The workspace of a call is what the library asks for, at every size."""
+    lib = _lib.load()
+    name = f"moddit_{op}_workspace_bytes"
+    asked = []
+    monkeypatch.setattr(lib, name, lambda *sizes: 4096)
+    monkeypatch.setattr(ops, "_workspace", lambda nbytes, device: asked.append(nbytes) or (None, 0))
+    q, k, v = _qkv(1, 1, 128, 128, 64, torch.bfloat16, False)
+    tiles = ops.mask_to_tiles(torch.ones((1, 2, 2), dtype=torch.bool, device="cuda"), 64)
+    ops._split_bytes.cache_clear()
+    try:
+        getattr(ops, op)(*((q, k, v) if op == "flash_fwd" else (q, k, v, tiles)))
+    finally:
+        ops._split_bytes.cache_clear()
+    assert asked == [4096]
