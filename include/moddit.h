@@ -101,7 +101,9 @@ int moddit_block_sparse_fwd(const void* q, const void* k, const void* v, void* o
  * then split each tile's key range over several workgroups, which leave fp32 partial
  * results in the workspace, and combine them in a second launch. *_workspace_bytes gives
  * the size such a call needs, 0 where it would not split; with a NULL workspace the calls
- * are the plain ones. The results differ from the plain call's by fp32 summation order.
+ * are the plain ones. Each piece of a split key range takes its weights against its own
+ * maximum before they are rounded to the storage type, so split and plain results agree to
+ * that rounding (unit roundoff 2^-8 bf16, 2^-11 fp16, relative to sum p |v|), not to fp32's.
  */
 int64_t moddit_flash_fwd_workspace_bytes(int batch, int heads, int q_len, int kv_len, int head_dim);
 int64_t moddit_block_sparse_fwd_workspace_bytes(int batch, int heads, int q_len, int head_dim,

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import functools
 import math
+import warnings
 from dataclasses import dataclass
 
 import torch
@@ -89,12 +90,15 @@ def _split_bytes(query: str, *sizes: int) -> int:
 
 def _workspace(nbytes: int, device):
     """(buffer, size) for a launch that can use `nbytes` of scratch: its own for each call, on
-    the current stream. Where the memory is not to be had, the launch runs without."""
+    the current stream. Where the memory is not to be had, the launch runs without, which takes
+    longer and rounds otherwise: it warns."""
     if nbytes <= 0:
         return None, 0
     try:
         return torch.empty(nbytes, device=device, dtype=torch.uint8), nbytes
     except torch.cuda.OutOfMemoryError:
+        warnings.warn(f"attention: no memory for {nbytes} bytes of scratch; the call runs on one "
+                      "workgroup per query tile", RuntimeWarning, stacklevel=4)
         return None, 0
 
 
@@ -141,12 +145,16 @@ def _attention(q, k, v, scale, return_lse, tiles: TileList | None, out=None):
 
 
 def flash_fwd(q, k, v, softmax_scale=None, return_lse=True, out=None):
-    """Dense attention over all keys; returns (O (B,H,Sq,D), LSE (B,H,Sq) fp32 or None)."""
+    """Dense attention over all keys; returns (O (B,H,Sq,D), LSE (B,H,Sq) fp32 or None).
+
+    A call with few query rows shares each row's keys among several workgroups, through scratch
+    of its own; without the memory for it (a RuntimeWarning) it takes longer and its results
+    agree to the rounding of P to the storage type."""
     return _attention(q, k, v, softmax_scale, return_lse, None, out)
 
 
 def block_sparse_fwd(q, k, v, tiles: TileList, softmax_scale=None, return_lse=False, out=None):
-    """Attention restricted to the active key tiles of `tiles`."""
+    """Attention restricted to the active key tiles of `tiles` (scratch as in `flash_fwd`)."""
     return _attention(q, k, v, softmax_scale, return_lse, tiles, out)
 
 

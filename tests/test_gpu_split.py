@@ -127,3 +127,24 @@ def test_the_library_decides_what_splits(op, monkeypatch):
     finally:
         ops._split_bytes.cache_clear()
     assert asked == [4096]
+
+
+def test_without_memory_for_scratch(monkeypatch):
+    """A call whose scratch cannot be had warns and returns the unsplit launch's result."""
+    q, k, v = _qkv(1, 2, 256, 4096, 128, torch.bfloat16, False)
+    with monkeypatch.context() as mp:
+        mp.setattr(ops, "_workspace", lambda nbytes, device: (None, 0))
+        plain, plain_lse = ops.flash_fwd(q, k, v)
+    split, _ = ops.flash_fwd(q, k, v)
+    assert not torch.equal(split, plain)
+    real = torch.empty
+
+    def empty(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.cuda.OutOfMemoryError("no scratch")
+        return real(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    with pytest.warns(RuntimeWarning, match="scratch"):
+        out, lse = ops.flash_fwd(q, k, v)
+    assert torch.equal(out, plain) and torch.equal(lse, plain_lse)
