@@ -129,12 +129,13 @@ __global__ __launch_bounds__(kMtsThreads) void mts_kernel(MtsParams p) {
 // loop is unrolled by 8), the one that crosses to the next lane moves by a wave shift, and
 // the one that leaves the last lane is stored to LDS. Nothing is reduced across lanes, and
 // no atomic is used: with 23 LDS atomics per 8 x 16 cells and global atomics per tile, which
-// this replaced, the map took 62 us at n = 1800 x 24 (155.5 MB) and, where rows are not
-// 16-byte aligned, 85 us at n = 275 x 48 (7 MB, 96 workgroups), plus 9 us of clearing and
-// finishing launches; now 47.5 (3.3 TB/s) and 12 us, plus 7.3 and 4.7 us for the sums. It
-// issues 41 VALU instructions per row of 64 x 8 cells, half of them fp64, on three waves
-// per SIMD (148 VGPRs; held to 128 it spills and takes 89 us); a second register stage of
-// loads gains nothing.
+// this replaced, both launches took 60 us at n = 1800 x 24 (155.5 MB) and, where rows are not
+// 16-byte aligned, 67 us at n = 275 x 48 (7 MB); 51 (3.0 TB/s) and 13.5 us now. It issues 41
+// VALU instructions per row of 64 x 8 cells, half of them fp64, on four waves per SIMD (112
+// VGPRs); a second register stage of loads gains nothing. Loads that would pass the map's end
+// are moved back and shifted (edge_row); read cell by cell, as the last rows of a map and all
+// of a small one were at first, 16 x 16 blocks x 24 heads took 23.7 us (15.2 with the atomics,
+// 12.3 now).
 //
 // Exactness: every finite fp16 value is a multiple of 2^-24 below 2^16, so any sum of at
 // most 8192 of them needs at most 53 significant bits and is exact in fp64 in any order; a
@@ -253,57 +254,61 @@ __global__ __launch_bounds__(kMtsTileThreads, 3) void mts_tile_kernel(Mts1Params
     leaving = lane == row ? out : leaving;
     edge = wave_shift_up(edge);
   };
+  // the lane's cells of a row near the map's end or past it (zeros): the 16 bytes that end with
+  // the map instead of those past its end, shifted into place
+  auto edge_row = [&](int r) -> u32x4 {
+    u32x4 w = u32x4{};
+    if (r >= n) return w;
+    const int64_t at = head0 + static_cast<int64_t>(r) * n + (c0 < n ? c0 : 0);
+    if (cells >= kMtsCols) {
+      const int64_t from = at < cells - kMtsCols ? at : cells - kMtsCols;
+      const int drop = static_cast<int>(at - from);  // 0..7 cells
+      __builtin_memcpy(&w, p.map + from, 16);
+#pragma unroll
+      for (int b = 1; b < kMtsCols; b *= 2)  // right by 1, 2, 4 cells
+        if (drop & b) {
+          const uint64_t lo = w[0] | static_cast<uint64_t>(w[1]) << 32;
+          const uint64_t hi = w[2] | static_cast<uint64_t>(w[3]) << 32;
+          const uint64_t l = b == 4 ? hi : lo >> (16 * b) | hi << (64 - 16 * b);
+          const uint64_t h2 = b == 4 ? 0 : hi >> (16 * b);
+          w = u32x4{static_cast<uint32_t>(l), static_cast<uint32_t>(l >> 32),
+                    static_cast<uint32_t>(h2), static_cast<uint32_t>(h2 >> 32)};
+        }
+    } else {  // fewer cells than a load holds
+      for (int j = 0; j < kMtsCols; ++j)
+        if (at + j < cells) w[j >> 1] |= static_cast<uint32_t>(p.map[at + j]) << (16 * (j & 1));
+    }
+    return w;
+  };
 #pragma unroll 1
   for (int r8 = 0; r8 < kRows; r8 += 8) {
     const int r = rs + r8;
+    u32x4 raw[8];
     if (r + 8 <= n && head0 + static_cast<int64_t>(r + 7) * n + C0 + kMtsTileC <= cells) {
       // eight whole rows, 16 bytes per lane at any 2-byte address
-      u32x4 raw[8];
       const uint16_t* src = p.map + head0 + static_cast<int64_t>(r) * n + (c0 < n ? c0 : C0);
 #pragma unroll
       for (int rr = 0; rr < 8; ++rr) __builtin_memcpy(&raw[rr], src + static_cast<int64_t>(rr) * n, 16);
-#pragma unroll
-      for (int rr = 0; rr < 8; ++rr) {
-        raw[rr] &= keep;
-        add_row(raw[rr], rr);
-        step_down(dacc[(7 - rr) & 7], r8 + rr);
-        __builtin_amdgcn_sched_barrier(0);  // or all 64 cells are converted first, and spill
-      }
-      // The frame cells apart from the sums above, which stay free of branches. The empty asm
-      // keeps the compiler from moving the sums below these branches, and from carrying the
-      // 64 converted cells across them: either spills.
-#pragma unroll
-      for (int j = 0; j < kMtsCols; ++j) asm volatile("" : "+v"(cacc[j]), "+v"(dacc[j]));
-#pragma unroll
-      for (int rr = 0; rr < 8; ++rr) {
-        asm volatile("" : "+v"(raw[rr]));
-        add_frame(raw[rr], r + rr);
-      }
     } else {
-      // the last rows, cell by cell: nothing past the map's end is touched
-#pragma unroll 1
-      for (int rr = 0; rr < 8; ++rr) {
-        uint64_t lo = 0, hi = 0;
-        const uint16_t* src = p.map + head0 + static_cast<int64_t>(r + rr) * n + c0;
-        const int m = r + rr < n ? (n - c0 < kMtsCols ? n - c0 : kMtsCols) : 0;
-#pragma unroll 1
-        for (int j = 0; j < m; ++j) {
-          const uint64_t v = src[j];
-          if (j < 4)
-            lo |= v << (16 * j);
-          else
-            hi |= v << (16 * (j - 4));
-        }
-        const u32x4 raw = {static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32),
-                           static_cast<uint32_t>(hi), static_cast<uint32_t>(hi >> 32)};
-        add_row(raw, 0);
-        add_frame(raw, r + rr);
-        step_down(dacc[7], r8 + rr);
-        const double edge = dacc[7];
 #pragma unroll
-        for (int j = kMtsCols - 1; j > 0; --j) dacc[j] = dacc[j - 1];
-        dacc[0] = edge;
-      }
+      for (int rr = 0; rr < 8; ++rr) raw[rr] = edge_row(r + rr);
+    }
+#pragma unroll
+    for (int rr = 0; rr < 8; ++rr) {
+      raw[rr] &= keep;
+      add_row(raw[rr], rr);
+      step_down(dacc[(7 - rr) & 7], r8 + rr);
+      __builtin_amdgcn_sched_barrier(0);  // or all 64 cells are converted first, and spill
+    }
+    // The frame cells apart from the sums above, which stay free of branches. The empty asm
+    // keeps the compiler from moving the sums below these branches, and from carrying the
+    // 64 converted cells across them: either spills.
+#pragma unroll
+    for (int j = 0; j < kMtsCols; ++j) asm volatile("" : "+v"(cacc[j]), "+v"(dacc[j]));
+#pragma unroll
+    for (int rr = 0; rr < 8; ++rr) {
+      asm volatile("" : "+v"(raw[rr]));
+      add_frame(raw[rr], r + rr);
     }
   }
   // after the last row's shift, register j of lane l holds the diagonal of column 8l + j - 1
