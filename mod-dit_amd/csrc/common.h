@@ -81,9 +81,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 struct Bf16 {
   typedef bf16x8 vec8;
   typedef __bf16 elem;
-  static __device__ __forceinline__ f32x16 mma(vec8 a, vec8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-  }
   static __device__ __forceinline__ f32x4 mma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
@@ -102,9 +99,6 @@ struct Bf16 {
 struct Fp16 {
   typedef f16x8 vec8;
   typedef _Float16 elem;
-  static __device__ __forceinline__ f32x16 mma(vec8 a, vec8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-  }
   static __device__ __forceinline__ f32x4 mma16(vec8 a, vec8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
   }
@@ -155,23 +149,6 @@ __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) {
 __device__ __forceinline__ uint16_t u16_at(const u32x4& v, int i) {
   const uint32_t w = v[i >> 1];
   return static_cast<uint16_t>((i & 1) ? (w >> 16) : (w & 0xffffu));
-}
-
-// ---------------------------------------------------------------------------------
-// Buffer loads. A raw buffer resource covers one tensor slice; offsets are 32-bit
-// bytes. The VGPR offset (plus the instruction offset) is range-checked against
-// `bytes`: out-of-range 16-byte loads return zeros instead of touching memory. The
-// SGPR offset is not range-checked, so it may only carry offsets known to be in range.
-// ---------------------------------------------------------------------------------
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), static_cast<short>(0),
-                                           static_cast<int>(bytes), 0x00020000);
-}
-
-__device__ __forceinline__ u32x4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t voff,
-                                            uint32_t soff) {
-  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                       r, static_cast<int>(voff), static_cast<int>(soff), 0));
 }
 
 // ---------------------------------------------------------------------------------
