@@ -16,10 +16,10 @@
 // limit). Its price, two queries per lane and with them twice the row reductions, is kept
 // off most tiles: a lane compares its own scores with the running max, and the row max is
 // exchanged and moved only where one of them lies far above it (settle). Against the 32x32x16
-// kernel with a max per tile, on structured inputs: dense 24 heads x 115,200, D = 128 150.5 ->
-// 144.3 ms; block-sparse 40 x 69,120 20.5 -> 19.7 ms; 48 x 17,776, D = 64 1.51 -> 1.40 ms.
+// kernel with a max per tile, on structured inputs: dense 24 heads x 115,200, D = 128 155.9 ->
+// 146.5 ms; block-sparse 40 x 69,120 21.3 -> 20.4 ms; 48 x 17,776, D = 64 1.55 -> 1.44 ms.
 // Weighing a tile against the max as it is, and computing it again where that overflows, takes
-// the lanes' max off too (143.2, 19.8 and 1.45 ms) but costs peaked rows up to 40 %.
+// the lanes' max off too (147.1, 20.8 and 1.46 ms) but costs peaked rows up to 40 %.
 //
 // K and V tiles go straight from HBM into LDS (buffer_load ... lds, no register
 // staging), both row-major with an XOR swizzle on 16-byte chunks that keeps the operand
@@ -300,6 +300,21 @@ __global__ __launch_bounds__(kThreads, attn_waves(D, kMap)) __attribute__((amdgp
         s[kb][0] = E::mma16(a, qf[0][c], s[kb][0]);
         s[kb][1] = E::mma16(a, qf[1][c], s[kb][1]);
       }
+    }
+    // D = 128: K reads four fragments ahead of their products, one per two products. Left to
+    // itself the compiler issues most reads right before their use, and each pair of them is
+    // waited for: with it, 128 to 256 workgroups of 64 to 256 tiles took 2-6 % longer (4 heads x
+    // 4,096 tokens, all tiles: 90 against 86 us), exact rows 3-4 %, and at the power limit 1-2 %
+    // (dense 24 x 115,200: 147.9 against 146.5 ms). 6 to 12 ahead are no better. D = 64 spills.
+    if constexpr (D == 128) {
+      constexpr int kReads = 4 * kKC, kAhead = 4;
+      __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);  // 0x100: LDS reads
+#pragma unroll
+      for (int i = 0; i < kReads - kAhead; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);     // 0x008: MFMAs
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * kAhead, 0);
     }
   };
   // O += P V: of its 2 kDB steps in the order (t, db), [i0, i1)

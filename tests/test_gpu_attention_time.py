@@ -1,5 +1,6 @@
 """Times of bf16/fp16 attention calls relative to each other, in one process (GPU): what
-neither the scores' spread nor one more workgroup per CU may cost."""
+neither the scores' spread nor one more workgroup per CU may cost, and a wider head only so
+much."""
 import pytest
 import torch
 
@@ -53,3 +54,18 @@ def test_four_workgroups_share_a_cu_at_d64():
     t6, t8 = one(6), one(8)
     print(f"6 heads {t6:.1f} us, 8 heads {t8:.1f} us", flush=True)
     assert t8 <= 1.2 * t6, (t6, t8)
+
+
+def test_one_workgroup_per_cu_waits_little_for_k():
+    """Launches of one workgroup per two CUs, 64 key tiles each, where nothing hides a wait: twice
+    the products and K reads at d = 128 (measured 1.26 of the time at d = 64; 1.40 where each
+    read of K was waited for)."""
+    def one(D):
+        q, k, v = _qkv(4, 4096, D)
+        mask = torch.ones((4, 64, 64), dtype=torch.bool, device="cuda")
+        tiles = ops.mask_to_tiles(mask, 64)
+        return _us(lambda: ops.block_sparse_fwd(q, k, v, tiles))
+
+    t64, t128 = one(64), one(128)
+    print(f"{t64:.1f} us at d = 64, {t128:.1f} us at d = 128", flush=True)
+    assert t128 <= 1.33 * t64
