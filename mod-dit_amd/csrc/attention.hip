@@ -738,10 +738,10 @@ int launch_attention(const AttnParams& p, int batch, hipStream_t stream) {
 // lengths are known on the device only: a block-sparse list is taken to hold a quarter of its
 // capacity. On those shapes the choice is never slower than no split, on average 3.5 % from
 // the best of 1..32 pieces and at worst 25 % (sweeps of 16 key tiles, which are kept at two
-// pieces): 256 text rows x 24 heads over 29,019 keys, D = 128 (48 tiles): 614 us unsplit,
-// 129 in 10 pieces; over 115,419 keys 2,414 and 455 us; 4,096 tokens x 2 heads, D = 64 (64
-// tiles): 66 and 29 us. Two tiles per CU no longer gain (432 tiles of 36 key tiles: 46 us
-// unsplit, 58 us in two). A list that holds less than a twentieth of its capacity loses the
+// pieces): 256 text rows x 24 heads over 29,019 keys, D = 128 (48 tiles): 590 us unsplit,
+// 135 in 10 pieces; over 115,419 keys 2,318 and 465 us; 4,096 tokens x 2 heads, D = 64 (64
+// tiles): 66 and 29 us. Two tiles per CU no longer gain (432 tiles of 36 key tiles: 47 us
+// unsplit, 59 us in two). A list that holds less than a twentieth of its capacity loses the
 // second launch, 4 us (32 tiles of one entry, D = 64: 13.4 -> 17.5 us a call).
 constexpr int kMaxSplit = 64;
 // Key tiles per piece at the least: below 16 key tiles the second launch costs a dense call
