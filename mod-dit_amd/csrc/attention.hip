@@ -114,7 +114,7 @@ __device__ __forceinline__ int swz_v(int key) { return 2 * ((key / (128 / D)) % 
 // 2.82e-4). 4 would take another 4-5 % off, and costs rows whose deviation is 2 to 8 2-3 %.
 constexpr float kRescaleSlack = 6.0f;
 
-// Waves per SIMD that the registers are held to. D = 128 takes 211-227 (two waves). D = 64 fits
+// Waves per SIMD that the registers are held to. D = 128 takes 212-228 (two waves). D = 64 fits
 // four in 124-128 (left alone, up to 134; the aligned dense kernel keeps seven invariants of
 // its last tile in scratch), the fused map three. Where a launch has four workgroups per CU,
 // three waves leave a quarter of them to a second round: 8 heads x 16,384, exact rows, a
@@ -461,10 +461,10 @@ __global__ __launch_bounds__(kThreads, attn_waves(D, kMap)) __attribute__((amdgp
     if (act_cur && act_next) {
       f32x4 s[4][2];
       // The P.V steps lie where something else waits. D = 128: some under the max of the new
-      // scores, the others under their weights (10 and 6 of 16; all before: 1-2 % slower where
-      // power does not bound, all after: 2-6 % on large calls); left to itself the scheduler
-      // spreads the S products over them, and the softmax waits. D = 64: half the products and
-      // as much softmax, which starts sooner after P.V; four waves cover the rest.
+      // scores, the others under their weights (10 and 6 of 16; 12 and 4: 3 % slower on small
+      // launches; 16 and 0: 4-7 % there and 3 % on large dense calls); left to itself the
+      // scheduler spreads the S products over them, and the softmax waits. D = 64: half the
+      // products and as much softmax, which starts sooner after P.V; four waves cover the rest.
       constexpr int kUnderMax = 10;
       if constexpr (D == 64) pv(vs, pb);
       qk(ks1, s);
